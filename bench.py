@@ -103,7 +103,8 @@ def kernel_name(form: str, shape, nl: int) -> str:
     kind, nk, ch, pers = shape
     flag = "true" if pers else "false"
     if form == "fp64":
-        return (f"los_sweep_exact<{nk}, {nl}, {flag}>" if kind == 1 else
+        return (f"los_window_exact<{nl}, {ch}, {64 // nk}>" if kind == 3 else
+                f"los_sweep_exact<{nk}, {nl}, {flag}>" if kind == 1 else
                 f"los_klane_exact<{nl}, {ch}>" if kind == 2 else f"los_integrate_exact<{nl}>")
     pol = POLICY[form]
     if kind == 1:
@@ -719,6 +720,8 @@ def main(argv=None):
         res["tile_shape"] = ({"kernel": "sweep", "nk": nk, "persistent": pers,
                               "j_pairs": bool(form != "fp32c" or ch == 1)} if kind == 1 else
                              {"kernel": "k-lane", "l_per_lane": ch} if kind == 2 else
+                             {"kernel": "window", "k3_per_wave": nk, "l_per_wave": ch}
+                             if kind == 3 else
                              {"kernel": "workgroup per k3"} if form == "fp64" else
                              {"kernel": "stream", "nk": nk, "ch": ch, "persistent": pers})
         return res, out, tt2, tt_out

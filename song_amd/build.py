@@ -25,6 +25,7 @@ C_SOURCES = ["los_special.c", "los_lm.c", "los_bessel2.c", "los_scenario.c", "lo
 HIP_SOURCES = [
     ("los_engine.hip", []),
     ("los_kernels_exact.hip", ["-ffp-contract=off"]),
+    ("los_kernels_window.hip", ["-ffp-contract=off"]),
     ("los_kernels_fast.hip", []),
     ("los_serve.hip", []),
     ("los_bessel2_gpu.hip", ["-ffp-contract=off"]),

@@ -9,6 +9,7 @@
 #define LOS_MAX_MI 6      /* entries of the m-list */
 #define LOS_NC_MAX 256    /* coarse k3 values per pair handled by the spline kernel */
 #define LOS_EXACT_BLOCK_MAX 512 /* (l,m) lanes per workgroup of the exact LOS kernel */
+#define LOS_WIN_W 32      /* x points of a J row's window in LDS (window kernels) */
 #define LOS_BUF_MAX 0xFFFFF000u /* largest table read through a raw buffer resource */
 
 /* One (k1,k2) pair as laid out on the device. */
@@ -136,6 +137,18 @@ typedef struct {
   const void *Jk;        /* J re-laid out [jt][L][lm][x] (FP64 or FP32) */
   const int *kgrp;       /* lane groups: NLB (l,m) offsets of one m per group, -1 padding */
   int k_ngrp;            /* number of lane groups */
+
+  /* window kernels (one fine k3 per lane, J windows in LDS) */
+  const int *wplan_off;  /* first window of each tile in wplan */
+  const int2 *wplan;     /* windows of a tile: {first step, 2 x first x point + partial},
+                            ended by {number of steps, 0} */
+  unsigned Jk_bytes;     /* size of the table at Jk (read with 32-bit byte offsets) */
+  const int *wgrp[2];    /* groups of (l,m) offsets of one m, -1 padding: of E and B, of T */
+  int wgrp_off[2][LOS_MAX_MI + 1]; /* first group of each m-list entry */
+  int *wix;              /* [rank / 64][t][64] index_x */
+  double *waj;           /* [rank / 64][t][64] a_J */
+  double *wsrc;          /* interpolated sources, per (field set, m) */
+  long wsrc_off[2][LOS_MAX_MI]; /* of E and B, of T */
 
   /* output blocks of the jobs */
   double *out;

@@ -76,10 +76,16 @@ static void free_batch(los_engine *e)
   dfree(e->dposjob);
   dfree(e->docol);
   dfree(e->djobs);
-  for (int i = 0; i < 5; ++i) {
+  for (int i = 0; i < LOS_TILE_SLOTS; ++i) {
     dfree(e->dtiles[i]);
+    dfree(e->dwplan_off[i]);
+    dfree(e->dwplan[i]);
+    dfree(e->dwtiles[i]);
     e->htiles[i].clear();
   }
+  dfree(e->dwix);
+  dfree(e->dwaj);
+  dfree(e->dwsrc);
   dfree(e->dspl);
   dfree(e->draw);
   dfree(e->dsrc);
@@ -112,7 +118,7 @@ static void free_tables(los_engine *e)
   }
   dfree(e->dJk);
   dfree(e->dJk32);
-  for (int gs = 0; gs < 3; ++gs) dfree(e->dkgrp[gs]);
+  for (int gs = 0; gs < LOS_KGRPS; ++gs) dfree(e->dkgrp[gs]);
   dfree(e->dxminp);
   dfree(e->dlm_of_lp);
   e->J_owner = nullptr;
@@ -274,6 +280,7 @@ static int build_tables(los_engine *e, const los_stage *st, double kmax_all, cha
 
   free_tables(e);
   e->hxmin = hxmin;
+  e->hminx = hminx;
   e->hm_of = hm;
   e->n_lp = n_lp;
   e->m_size = m_size;
@@ -290,11 +297,12 @@ static int build_tables(los_engine *e, const los_stage *st, double kmax_all, cha
     HIPCHK(hipMalloc((void **)&e->dJk, nJ * sizeof(double)), err);
     if (upload(e, e->dJk, hJk.data(), nJ * sizeof(double), err)) return _FAILURE_;
     // lane groups: for each m-list entry, the (l,m) offsets in l order, cut
-    // into groups of 1, 2 or 4
-    for (int gs = 0; gs < 3; ++gs) {
+    // into groups of 1, 2, 4 or 8
+    for (int gs = 0; gs < LOS_KGRPS; ++gs) {
       const int nlb = 1 << gs;
       std::vector<int> grp;
       for (int im = 0; im < m_size; ++im) {
+        e->kgrp_off[gs][im] = (int)grp.size() / nlb;
         std::vector<int> lms;
         for (int il = 0; il < n_l; ++il)
           if (im <= st->index_m_max[st->l[il]]) lms.push_back(st->lm_array[il][im]);
@@ -302,6 +310,7 @@ static int build_tables(los_engine *e, const los_stage *st, double kmax_all, cha
           for (int j = 0; j < nlb; ++j) grp.push_back(q + j < lms.size() ? lms[q + j] : -1);
       }
       e->kngrp[gs] = (int)grp.size() / nlb;
+      for (int im = m_size; im <= LOS_MAX_MI; ++im) e->kgrp_off[gs][im] = e->kngrp[gs];
       if (upload_vec(e, e->dkgrp[gs], grp, err)) return _FAILURE_;
     }
   }
@@ -354,7 +363,11 @@ void split_xcd(const std::vector<los_tile> &tiles, const std::vector<double> &po
   out[8] = nt;
 }
 
-int nk_slot(int nk) { return nk == 1 ? 0 : nk == 2 ? 1 : nk == 4 ? 2 : nk == 8 ? 3 : 4; }
+int nk_slot(int nk)
+{
+  return nk == 1 ? 0 : nk == 2 ? 1 : nk == 4 ? 2 : nk == 8 ? 3 : nk == 16 ? 4 : nk == 32 ? 5 : 6;
+}
+static int slot_nk(int slot) { return 1 << slot; }
 
 // Tiles of at most nk consecutive positions that never straddle two jobs
 // (job_end: one past the last position of each job, ascending).
@@ -367,6 +380,83 @@ std::vector<los_tile> make_tiles(const std::vector<int> &job_end, int nk)
     begin = end;
   }
   return t;
+}
+
+// Windows of the tiles of slot `slot` (window kernels): starting at a step, the
+// LOS_WIN_W - 1 x points that end at the index_x of the tile's largest k3, kept for
+// as many steps as hold the index_x of all its k3 (index_x falls with the
+// step). Where one step needs more points, the step has several windows, each
+// marked partial. No list is kept (and the tile size not offered) when the
+// steps need more than LOS_WIN_MOST windows on average: every window is a pass
+// over all lanes, and the other organisations gather only what they need.
+#define LOS_WIN_MOST 2
+#define LOS_WIN_DEAL 8 /* one round: 41 ms where eight take 30.0 (32 x 32 pairs, 96 l) */
+static int make_window_plan(los_engine *e, int slot, const std::vector<double> &kf,
+                            const std::vector<int> &forder, double xx_step, char *err)
+{
+  const std::vector<los_tile> &tiles = e->htiles[slot];
+  const std::vector<double> &t0mt = e->ht0mt;
+  const int ntau = e->ntau;
+  const int nt = (int)tiles.size();
+  std::vector<int> off(nt), alive(e->X + 1, 0);  // alive[x]: (l,m) live at x
+  for (int v : e->hminx)
+    if (v < e->X) alive[v]++;
+  for (int x = 1; x <= e->X; ++x) alive[x] += alive[x - 1];
+  std::vector<int2> win;
+  std::vector<double> before(nt + 1, 0.0);  // cost of the tiles before each
+  for (int q = 0; q < nt; ++q) {
+    off[q] = (int)win.size();
+    const double kmin = kf[forder[tiles[q].pos0]];
+    const double kmax = kf[forder[tiles[q].pos0 + tiles[q].npos - 1]];
+    auto ix = [&](double k, int t) { return (int)(k * t0mt[t] / xx_step); };
+    double c = 8.0 * e->n_lm;
+    int t = 0;
+    while (t < ntau) {
+      const int hi = ix(kmax, t), lo = ix(kmin, t);
+      const double live = alive[std::min(hi, e->X)];
+      if (live == 0) break;
+      const int t0 = t;
+      if (hi - lo < LOS_WIN_W - 1) {
+        const int x0 = std::max(0, hi - LOS_WIN_W + 2);
+        win.push_back(int2{t, 2 * x0});
+        while (++t < ntau && ix(kmin, t) >= x0) {}
+        c += (t - t0 + 1) * live;
+      } else {
+        for (int x0 = lo; x0 <= hi; x0 += LOS_WIN_W - 1) {
+          win.push_back(int2{t, 2 * x0 + 1});
+          c += 2 * live;
+        }
+        ++t;
+      }
+      if (win.size() > (size_t)LOS_WIN_MOST * nt * ntau) return _SUCCESS_;
+    }
+    win.push_back(int2{ntau, 0});
+    before[q + 1] = before[q] + c;
+  }
+  // the tiles dealt to the XCDs in LOS_WIN_DEAL rounds of 8 runs of neighbouring
+  // tiles of about equal cost: a run is about what an XCD holds at once (its L2
+  // serves the run's J rows), and every XCD gets runs from all over the k3 range
+  std::vector<std::vector<int>> of(8);
+  for (int c = 0, q = 0; c < 8 * LOS_WIN_DEAL; ++c) {
+    const int x = (c / 8) % 2 ? 7 - c % 8 : c % 8;
+    const double goal = before[nt] * (c + 1) / (8 * LOS_WIN_DEAL);
+    while (q < nt && (c == 8 * LOS_WIN_DEAL - 1 || before[q + 1] <= goal)) of[x].push_back(q++);
+  }
+  std::vector<los_tile> wt;
+  std::vector<int> woff;
+  for (int x = 0; x < 8; ++x) {
+    e->wxcd[slot][x] = (int)wt.size();
+    for (int q : of[x]) {
+      wt.push_back(tiles[q]);
+      woff.push_back(off[q]);
+    }
+  }
+  e->wxcd[slot][8] = (int)wt.size();
+  off = woff;
+  if (upload_vec(e, e->dwtiles[slot], wt, err)) return _FAILURE_;
+  if (upload_vec(e, e->dwplan_off[slot], off, err) || upload_vec(e, e->dwplan[slot], win, err))
+    return _FAILURE_;
+  return _SUCCESS_;
 }
 
 extern "C" int los_engine_load_stage(los_engine *e, const los_stage *st, const int *pk1,
@@ -590,16 +680,17 @@ extern "C" int los_engine_load_stage(los_engine *e, const los_stage *st, const i
   jobs[0].ttT = st->index_tt2_T;
   jobs[0].ttE = st->index_tt2_E;
   jobs[0].ttB = st->index_tt2_B;
-  for (int i = 0; i < 5; ++i) {
+  for (int i = 0; i < LOS_TILE_SLOTS; ++i) {
     // tiles never straddle two chunks; chunk_tile[i] holds each chunk's first tile
     e->htiles[i] = make_tiles(std::vector<int>(e->chunk_pos.begin() + 1, e->chunk_pos.end()),
-                              i < 4 ? 1 << i : 64);
+                              slot_nk(i));
     e->chunk_tile[i].assign(e->n_chunk + 1, (int)e->htiles[i].size());
     for (int c = 0, t = 0; c < e->n_chunk; ++c) {
       while (t < (int)e->htiles[i].size() && e->htiles[i][t].pos0 < e->chunk_pos[c]) ++t;
       e->chunk_tile[i][c] = t;
     }
     if (upload_vec(e, e->dtiles[i], e->htiles[i], err)) return _FAILURE_;
+    if (i >= 4 && make_window_plan(e, i, kf, forder, st->xx_step, err)) return _FAILURE_;
   }
   if (upload_vec(e, e->dposjob, posjob, err) || upload_vec(e, e->docol, forder, err) ||
       upload_vec(e, e->djobs, jobs, err))
@@ -743,19 +834,31 @@ bool sweep_fits(const los_engine *e, int form, const los_shape &sh)
   return bytes <= (double)LOS_BUF_MAX;
 }
 
+// Whether the window kernels can take the loaded batch in tiles of kt k3.
+static bool window_fits(const los_engine *e, int kt)
+{
+  return e->loaded && !e->serving && !e->cubic_J && e->n_chunk == 1 && e->F > 0 &&
+         e->dwplan[nk_slot(kt)] != nullptr && (long)e->ntau * LOS_MAX_L * 2 * 512 <= INT_MAX &&
+         (e->P.has_E || !e->P.has_B) &&
+         (double)e->nJk * sizeof(double) <= (double)LOS_BUF_MAX && (!e->P.has_B || e->P.jEB >= 0) &&
+         los_window_rows_fit(e->P.has_T, e->P.has_E || e->P.has_B, e->P.LmaxT, e->P.LmaxP);
+}
+
 // Candidate kernel shapes of a form: the plain FP64 form has its
 // one-workgroup-per-k3 kernel (kind 0), the sweep (kind 1) and the k-lane
 // kernel (kind 2), all bit-identical to the reference; the fast forms every
 // stream, sweep and k-lane shape that fits.
 static int form_shapes(const los_engine *e, int form, los_shape *out, int cap)
 {
-  los_shape all[48];
+  los_shape all[64];
   int n = 0;
   if (form == LOS_FORM_FP64) {
     all[n++] = los_shape{0, 1, 0, 0};
     for (int nk = 1; nk <= 8; nk *= 2)
       for (int p = 0; p < 2; ++p) all[n++] = los_shape{1, nk, 0, p};
     for (int b = 1; b <= 4; b *= 2) all[n++] = los_shape{2, 64, b, 0};
+    for (int kt = 64; kt >= 16; kt /= 2)
+      if (window_fits(e, kt)) all[n++] = los_shape{3, kt, 8, 0};
   } else {
     n = los_shapes(form == LOS_FORM_FP32C, e->loaded ? e->P.tp2_size : 1, all, 48);
   }
@@ -792,6 +895,23 @@ int enqueue_los_params(los_engine *e, const los_shape *sh, los_params *P, hipStr
       HIPCHK(los_launch_klane_exact(P, sh->ch, s), err);
     else
       HIPCHK(los_launch_klane(fp32, P, sh->ch, s), err);
+    return _SUCCESS_;
+  }
+  if (sh->kind == 3) {
+    // sh->ch = 8 (l,m) offsets a wave, 4 where it holds the rows of two J types
+    const int slot = nk_slot(sh->nk), gs[2] = {P->has_B ? 2 : 3, 3};
+    P->Jk = e->dJk;
+    P->Jk_bytes = (unsigned)(e->nJk * sizeof(double));
+    for (int set = 0; set < 2; ++set) {
+      P->wgrp[set] = e->dkgrp[gs[set]];
+      for (int im = 0; im <= LOS_MAX_MI; ++im)
+        P->wgrp_off[set][im] = e->kgrp_off[gs[set]][im];
+    }
+    P->wplan_off = e->dwplan_off[slot];
+    P->wplan = e->dwplan[slot];
+    P->tiles = e->dwtiles[slot];
+    std::copy(e->wxcd[slot], e->wxcd[slot] + 9, P->xcd_tile);
+    HIPCHK(los_launch_window_exact(P, sh->nk, sh->ch, s), err);
     return _SUCCESS_;
   }
   if (e->form == LOS_FORM_FP64 && sh->kind == 1) {
@@ -857,6 +977,8 @@ static int enqueue_tables(los_engine *e, const los_shape *sh, char *err, int f_b
       HIPCHK(los_launch_klane_prep_exact(&e->P, e->stream), err);
     else
       HIPCHK(los_launch_klane_prep(fp32, &e->P, e->stream), err);
+  } else if (sh->kind == 3) {
+    HIPCHK(los_launch_window_prep(&e->P, e->stream), err);
   }
   return _SUCCESS_;
 }
@@ -1013,9 +1135,35 @@ int ensure_klane(los_engine *e, const los_shape *sh, char *err)
   return _SUCCESS_;
 }
 
+// Device tables a window shape needs (allocated outside any capture).
+static int ensure_window(los_engine *e, const los_shape *sh, char *err)
+{
+  if (sh == nullptr || sh->kind != 3) return _SUCCESS_;
+  if (e->dwsrc) return _SUCCESS_;
+  const size_t n = (size_t)e->P.k_npad * e->ntau;
+  size_t rows = 0;
+  for (int set = 0; set < 2; ++set)
+    for (int mi = 0; mi < e->P.m_size; ++mi) {
+      e->P.wsrc_off[set][mi] = (long)(rows * n);
+      if (set ? !e->P.has_T : !(e->P.has_E || e->P.has_B)) continue;
+      const int nr = los_window_jrows(std::max(e->P.LmaxT, e->P.LmaxP) + 1,
+                                      set ? e->P.LmaxT : e->P.LmaxP, e->P.m_of_mi[mi]);
+      rows += (size_t)nr * (set || !e->P.has_B ? 1 : 2);
+    }
+  HIPCHK(hipMalloc((void **)&e->dwix, n * sizeof(int)), err);
+  HIPCHK(hipMalloc((void **)&e->dwaj, n * sizeof(double)), err);
+  HIPCHK(hipMalloc((void **)&e->dwsrc, std::max<size_t>(1, rows * n) * sizeof(double)), err);
+  e->P.wix = e->dwix;
+  e->P.waj = e->dwaj;
+  e->P.wsrc = e->dwsrc;
+  return _SUCCESS_;
+}
+
 static int ensure_tables(los_engine *e, const los_shape *sh, char *err)
 {
-  return ensure_sweep(e, sh, err) || ensure_klane(e, sh, err) ? _FAILURE_ : _SUCCESS_;
+  return ensure_sweep(e, sh, err) || ensure_klane(e, sh, err) || ensure_window(e, sh, err)
+             ? _FAILURE_
+             : _SUCCESS_;
 }
 
 int ensure_j32(los_engine *e, char *err)
@@ -1031,17 +1179,18 @@ int ensure_j32(los_engine *e, char *err)
 }
 
 // Autotuner cache: best shape per (form, (l,m) count, source types, sources L,
-// time steps, fine-k3 count rounded to a power of two).
-typedef std::tuple<int, int, int, int, int, int, int> tune_key;
+// time steps, fine-k3 count rounded to a power of two, window tiles that fit).
+typedef std::tuple<int, int, int, int, int, int, int, int, int> tune_key;
 static std::map<tune_key, los_shape> g_tuned;
 static std::mutex g_tuned_mu;
 
 static tune_key key_of(const los_engine *e)
 {
-  int fb = 0;
+  int fb = 0, windows = 0;  // windows: the tile sizes the batch's k3 spacing allows
   while ((1 << fb) < e->F) ++fb;
+  for (int kt = 16; kt <= 64; kt *= 2) windows |= window_fits(e, kt) ? kt : 0;
   return tune_key(e->form, e->n_lm, e->P.tp2_size, std::max(e->P.LmaxT, e->P.LmaxP), e->ntau, fb,
-                  e->cubic_J ? 1 : 0);
+                  e->cubic_J ? 1 : 0, e->serving ? 1 : 0, windows);
 }
 
 extern "C" int los_engine_autotune(los_engine *e, int reps, char *err)
@@ -1065,7 +1214,7 @@ extern "C" int los_engine_autotune(los_engine *e, int reps, char *err)
   }
   if (reps < 1) reps = 1;
   if (ensure_j32(e, err)) return _FAILURE_;
-  los_shape all[48], cand[48];
+  los_shape all[64], cand[48];
   const int na = form_shapes(e, form, all, 48);
   int nc = 0;
   for (int i = 0; i < na; ++i)
@@ -1118,6 +1267,7 @@ extern "C" int los_engine_set_shape(los_engine *e, int form, int kind, int nk, i
   for (int i = 0; i < nc; ++i)
     if (cand[i].kind == kind &&
         (kind == 2   ? cand[i].ch == ch
+         : kind == 3 ? (cand[i].nk == nk && cand[i].ch == ch)
          : kind == 1 ? (cand[i].nk == nk && cand[i].persistent == (persistent != 0) &&
                         cand[i].ch == ch)
                      : (form == LOS_FORM_FP64 ||

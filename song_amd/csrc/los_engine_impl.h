@@ -43,7 +43,14 @@ extern "C" hipError_t los_launch_klane_prep(int fp32, const los_params *P, hipSt
 extern "C" hipError_t los_launch_klane(int fp32, const los_params *P, int nlb, hipStream_t s);
 extern "C" hipError_t los_launch_klane_prep_exact(const los_params *P, hipStream_t s);
 extern "C" hipError_t los_launch_klane_exact(const los_params *P, int nlb, hipStream_t s);
+extern "C" hipError_t los_launch_window_prep(const los_params *P, hipStream_t s);
+extern "C" hipError_t los_launch_window_exact(const los_params *P, int kt, int nl, hipStream_t s);
+extern "C" int los_window_jrows(int NL, int Lmax, int m);
+extern "C" int los_window_rows_fit(int has_T, int has_P, int LmaxT, int LmaxP);
 extern "C" hipError_t los_launch_round_j32(const double *src, float *dst, long n, hipStream_t s);
+
+#define LOS_TILE_SLOTS 7 /* tile sizes a loaded batch is cut into */
+#define LOS_KGRPS 4      /* lane groups of 1, 2, 4, 8 (l,m) offsets */
 
 struct los_engine {
   int device = 0;
@@ -60,7 +67,7 @@ struct los_engine {
   int chunks_forced = 0;              // chunk count set by the caller (0: one chunk)
   int n_chunk = 1;                    // chunk count of the loaded batch
   std::vector<int> chunk_pair, chunk_f, chunk_pos;  // [n_chunk + 1] boundaries
-  std::vector<int> chunk_tile[5];     // [n_chunk + 1] tile boundaries per tile-size slot
+  std::vector<int> chunk_tile[LOS_TILE_SLOTS];     // [n_chunk + 1] tile boundaries per tile-size slot
 
   // projection tables (resident across loads)
   const void *J_owner = nullptr;
@@ -73,6 +80,7 @@ struct los_engine {
   int X = 0, L_size = 0, J_size = 0, n_lm = 0;
   int minx_all = INT_MAX;  // smallest first-live x index over all rows in use
   std::vector<int> hxmin;  // host copy of xmin [jt][L][lm]
+  std::vector<int> hminx;  // smallest first-live x index of each (l,m) offset's rows
   std::vector<int> hm_of;  // m of each (l,m) offset
   std::vector<double> ht0mt;  // tau0 - tau of the loaded time grid
   // the same table laid out for the sweep kernels: [jt][L][x][lp], lane slot
@@ -93,8 +101,9 @@ struct los_engine {
   double *dJk = nullptr;
   float *dJk32 = nullptr;
   size_t nJk = 0;
-  int *dkgrp[3] = {nullptr, nullptr, nullptr};  // lane groups of 1, 2, 4 (l,m) offsets
-  int kngrp[3] = {0, 0, 0};
+  int *dkgrp[LOS_KGRPS] = {};  // lane groups of 1, 2, 4, 8 (l,m) offsets
+  int kngrp[LOS_KGRPS] = {};
+  int kgrp_off[LOS_KGRPS][LOS_MAX_MI + 1] = {};  // first group of each m-list entry
   double J_window_bytes = 0;
 
   // time grid
@@ -108,8 +117,8 @@ struct los_engine {
   int *dfpair = nullptr, *dfsrc = nullptr, *dfbr = nullptr, *dforder = nullptr;
   int *dposjob = nullptr, *docol = nullptr;
   los_job *djobs = nullptr;
-  std::vector<los_tile> htiles[5];     // tiles of 1, 2, 4, 8, 64 positions
-  los_tile *dtiles[5] = {nullptr, nullptr, nullptr, nullptr, nullptr};
+  std::vector<los_tile> htiles[LOS_TILE_SLOTS];  // tiles of 1, 2, 4, .. 64 positions
+  los_tile *dtiles[LOS_TILE_SLOTS] = {};
   double *draw = nullptr, *dsrc = nullptr, *ddd = nullptr, *dout = nullptr;
   long src_total = 0;
   int nc_max = 0;
@@ -135,6 +144,15 @@ struct los_engine {
   void *dkixa = nullptr, *dksrc = nullptr;  // tables of the k-lane kernels
   int klane_form = -1;                   // form whose tables they hold (-1: none)
   size_t klane_bytes = 0;
+
+  // window kernels: windows of the tiles of 16 to 64 positions, made with the batch; no list where a tile size's k3 lie too far apart
+  int *dwplan_off[LOS_TILE_SLOTS] = {};
+  int2 *dwplan[LOS_TILE_SLOTS] = {};
+  los_tile *dwtiles[LOS_TILE_SLOTS] = {};  // the tiles as dealt to the XCDs
+  int wxcd[LOS_TILE_SLOTS][9] = {};        // first tile of each XCD
+  int *dwix = nullptr;                   // tables (plain FP64 form)
+  double *dwaj = nullptr, *dwsrc = nullptr;
+  bool serving = false;                  // tiles are made per launch (the job server)
 
   int n_cu = 256;
   int *dqueue = nullptr;               // work-queue counters of the persistent kernels

@@ -307,6 +307,7 @@ extern "C" int los_server_create_stage(int device, int form, double hbm_budget_b
     return _FAILURE_;
   }
   los_engine *e = S->e;
+  e->serving = true;  // tiles are cut per launch: shapes with per-batch tile lists are out
   // resident preparation: source re-layout and k3 spline, kernel shape, and the
   // per-(k3, tau) tables of a sweep shape
   const los_shape *sh = nullptr;
