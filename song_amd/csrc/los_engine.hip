@@ -857,11 +857,12 @@ static int form_shapes(const los_engine *e, int form, los_shape *out, int cap)
     for (int nk = 1; nk <= 8; nk *= 2)
       for (int p = 0; p < 2; ++p) all[n++] = los_shape{1, nk, 0, p};
     for (int b = 1; b <= 4; b *= 2) all[n++] = los_shape{2, 64, b, 0};
-    for (int kt = 64; kt >= 16; kt /= 2)
-      if (window_fits(e, kt)) all[n++] = los_shape{3, kt, 8, 0};
   } else {
     n = los_shapes(form == LOS_FORM_FP32C, e->loaded ? e->P.tp2_size : 1, all, 48);
   }
+  if (form != LOS_FORM_FP32C)
+    for (int kt = 64; kt >= 16; kt /= 2)
+      if (window_fits(e, kt)) all[n++] = los_shape{3, kt, 8, 0};
   int k = 0;
   for (int i = 0; i < n && k < cap; ++i) {
     // cubic interpolation of J: the plain FP64 sweep kernels only
@@ -911,7 +912,10 @@ int enqueue_los_params(los_engine *e, const los_shape *sh, los_params *P, hipStr
     P->wplan = e->dwplan[slot];
     P->tiles = e->dwtiles[slot];
     std::copy(e->wxcd[slot], e->wxcd[slot] + 9, P->xcd_tile);
-    HIPCHK(los_launch_window_exact(P, sh->nk, sh->ch, s), err);
+    if (e->form == LOS_FORM_FP64)
+      HIPCHK(los_launch_window_exact(P, sh->nk, sh->ch, s), err);
+    else
+      HIPCHK(los_launch_window_fma(P, sh->nk, sh->ch, s), err);
     return _SUCCESS_;
   }
   if (e->form == LOS_FORM_FP64 && sh->kind == 1) {

@@ -37,6 +37,8 @@
 // - Tiles of 64, 32 or 16 k3: the sparser the k3, the fewer share a window; the
 //   tuner picks (9,404 k3, T only, 48 l: 1.75, 0.89, 0.34 ms against the sweep
 //   kernel's 1.11 ms; 14,753 k3 up to 0.2/Mpc: 44.7, 26.6, 27.1 against 53.1 ms).
+// With FMA (11,178 k3, T+E+B, 96 l): 22.0, 14.3, 12.4 ms against 32.0 to 41.1 ms of
+// the sweep kernel's tiles.
 //
 // Tables, by blocks of 64 sorted ranks (r = 64 rb + lane), so that a wave's
 // stream through the time steps is contiguous:
@@ -89,82 +91,6 @@ __host__ __device__ static inline int win_jrows(int NL, int Lmax, int m)
 __device__ __forceinline__ int win_jrows(const los_params &P, int set, int m)
 {
   return win_jrows(max(P.LmaxT, P.LmaxP) + 1, set ? P.LmaxT : P.LmaxP, m);
-}
-
-// The tables of the window kernels. A workgroup makes 64 ranks x 64 time steps:
-// it reads the sources along tau (their layout in HBM) and writes along the
-// ranks through an LDS transpose.
-__global__ void __launch_bounds__(256) los_window_prep(los_params P)
-{
-  __shared__ double tile[64][65];
-  __shared__ long r_off[64];
-  __shared__ int r_nc[64];
-  __shared__ double r_aw[64], r_bw[64], r_ca[64], r_cb[64], r_h[64];
-  const int rb = blockIdx.x, r0 = rb * 64, t0 = blockIdx.y * 64;
-  const int tid = threadIdx.x, lane = tid & 63, grp = tid >> 6;
-  double kf = 0;
-  {
-    const int r = min(r0 + lane, P.F - 1);
-    const int f = P.korder[r];
-    kf = P.kf[f];
-    if (tid < 64) {
-      const los_pair pr = P.pairs[P.fpair[f]];
-      const int br = P.fbr[f];
-      const double *kc = P.kc + pr.kc_off;
-      const double ks = P.kf[P.fsrc[f]];
-      const double h = kc[br + 1] - kc[br];
-      const double bw = (ks - kc[br]) / h;
-      const double aw = 1 - bw;
-      r_off[tid] = pr.src_off + (long)br * P.ntau;
-      r_nc[tid] = pr.nc;
-      r_h[tid] = h;
-      r_aw[tid] = aw;
-      r_bw[tid] = bw;
-      r_ca[tid] = aw * aw * aw - aw;
-      r_cb[tid] = bw * bw * bw - bw;
-    }
-  }
-  for (int i = grp; i < 64; i += 4) {
-    const int t = t0 + i;
-    if (t >= P.ntau) break;
-    const double x = kf * P.t0mt[t];
-    const int ix = (int)(x / P.xx_step);
-    const long o = ((long)rb * P.ntau + t) * 64 + lane;
-    P.wix[o] = ix;
-    P.waj[o] = (P.xx[ix + 1] - x) / P.xx_step;
-  }
-  const int tr = min(t0 + lane, P.ntau - 1);
-  __syncthreads();
-  for (int set = 0; set < 2; ++set) {
-    if (set ? !P.has_T : !(P.has_E || P.has_B)) continue;
-    const int Lmax = set ? P.LmaxT : P.LmaxP, nf = set || !P.has_B ? 1 : 2;
-    for (int mi = 0; mi < P.m_size; ++mi) {
-      const int m = P.m_of_mi[mi], nr = win_jrows(P, set, m), rows = nr * nf;
-      double *out = P.wsrc + P.wsrc_off[set][mi] + (long)rb * P.ntau * rows * 64;
-      for (int row = 0; row < rows; ++row) {
-        const int L = Lmax - nr + 1 + row / nf;
-        const bool live = L >= m;
-        const int tp = !live ? 0 : set ? P.srcT[L][mi] : row % nf ? P.srcB[L][mi] : P.srcE[L][mi];
-#pragma unroll 4
-        for (int i = grp; i < 64; i += 4) {
-          const double *S = P.src + r_off[i] + (long)tp * r_nc[i] * P.ntau + tr;
-          double v;
-          if (P.cubic_k3) {
-            const double *D = P.dd + (S - P.src);
-            v = r_aw[i] * S[0] + r_bw[i] * S[P.ntau] +
-                (r_ca[i] * D[0] + r_cb[i] * D[P.ntau]) * r_h[i] * r_h[i] / 6.0;
-          } else {
-            v = r_aw[i] * S[0] + r_bw[i] * S[P.ntau];
-          }
-          tile[i][lane] = live ? v : 0.;
-        }
-        __syncthreads();
-        for (int i = grp; i < 64; i += 4)
-          if (t0 + i < P.ntau) out[((long)(t0 + i) * rows + row) * 64 + lane] = tile[lane][i];
-        __syncthreads();
-      }
-    }
-  }
 }
 
 // The lanes' positions and (l,m) of a wave.
@@ -423,9 +349,11 @@ __device__ __forceinline__ void win_item(const los_params &P, const WinWave &W, 
 // XCD's tiles, costliest first, then the l groups, so that the waves running
 // together read the sources of a few neighbouring tiles and the same stretch
 // of their J rows through the XCD's L2.
-template <int NL, int NLT, int G>
+// FMA tells the unit that instantiates it apart: the plain FP64 form (compiled
+// without contraction) or the FP64 form with FMA.
+template <bool FMA, int NL, int NLT, int G>
 __global__ void __launch_bounds__(64) __attribute__((amdgpu_waves_per_eu(2)))
-los_window_exact(los_params P)
+los_window(los_params P)
 {
   constexpr int KT = 64 / G;
   __shared__ alignas(16) double win[NL * NLT * LOS_WIN_W];  // windows of the wave's rows
@@ -477,8 +405,8 @@ static inline bool window_rows_fit(int has_T, int has_P, int LmaxT, int LmaxP)
 
 // P->tiles / P->xcd_tile: tiles of at most 64/G positions; P->wgrp: groups of NLT
 // (l,m) offsets, of NLT/2 for E and B with B sources.
-template <int NLT, int G>
-static hipError_t launch_window_exact(const los_params *P, hipStream_t s)
+template <bool FMA, int NLT, int G>
+static hipError_t launch_window(const los_params *P, hipStream_t s)
 {
   if (P->n_pos == 0 || P->n_lm_max == 0) return hipSuccess;
   long most = 0, groups = 0;
@@ -494,11 +422,23 @@ static hipError_t launch_window_exact(const los_params *P, hipStream_t s)
   switch ((P->LmaxT > P->LmaxP ? P->LmaxT : P->LmaxP) + 1) {
 #define LOS_WN(n)                                                                              \
   case n:                                                                                      \
-    hipLaunchKernelGGL((los_window_exact<n, NLT, G>), dim3((unsigned)grid), dim3(64), 0, s, *P); \
+    hipLaunchKernelGGL((los_window<FMA, n, NLT, G>), dim3((unsigned)grid), dim3(64), 0, s, *P); \
     break;
     LOS_WN(1) LOS_WN(2) LOS_WN(3) LOS_WN(4) LOS_WN(5) LOS_WN(6) LOS_WN(7) LOS_WN(8)
 #undef LOS_WN
     default: return hipErrorInvalidValue;
   }
   return hipGetLastError();
+}
+
+// kt fine k3 and nl (l,m) offsets per wave
+template <bool FMA>
+static hipError_t launch_window(const los_params *P, int kt, int nl, hipStream_t s)
+{
+  switch (kt * 64 + nl) {
+    case 64 * 64 + 8: return launch_window<FMA, 8, 1>(P, s);
+    case 32 * 64 + 8: return launch_window<FMA, 8, 2>(P, s);
+    case 16 * 64 + 8: return launch_window<FMA, 8, 4>(P, s);
+    default: return hipErrorInvalidValue;
+  }
 }

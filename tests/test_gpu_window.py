@@ -1,14 +1,14 @@
-"""The window kernels of the plain FP64 form (one fine k3 per lane, J windows in LDS) against
-the CPU oracle, bit for bit, where they can go wrong: every count of source multipoles L, rows
-below m, fields with fewer L than the other, T or E alone, odd l counts against the groups of 8
-and 4, k3 counts that leave partial tiles, one step over several windows, J rows with an
-index_xmin_J of their own, and a batch whose k3 lie too far apart.
+"""The window kernels (one fine k3 per lane, J windows in LDS) against the CPU oracle, the plain
+FP64 form bit for bit and the FMA-FP64 form at its bar, where they can go wrong: every count of
+source multipoles L, rows below m, fields with fewer L than the other, T or E alone, odd l
+counts against the groups of 8 and 4, k3 counts that leave partial tiles, one step over several
+windows, J rows with an index_xmin_J of their own, and a batch whose k3 lie too far apart.
 """
 import numpy as np
 import pytest
 
 from song_amd import lib as L
-from tests.conftest import run_oracle
+from tests.conftest import field_errors, run_oracle
 
 BASE = dict(has_T=1, has_E=1, m_list=[0, 1, 2], l_max_los_t=4, l_max_los_p=4, k_size=3,
             k_min=2e-3, k_max=0.01, k3_size=9, tau_size=37, l_size=9, l_max=140, dk_fine=2.5e-5,
@@ -53,6 +53,13 @@ def _run(cfg, oracle, overrides=()):
         eng.store(s)
         assert np.array_equal(s.gather(), ref), f"tile of {kt}"
         ran.append(kt)
+    eng.set_form(L.FORM_FP64_FAST)
+    tt2 = ref.size // int(s.k3_sizes()[:, 0].sum())
+    for kt in ran:  # the same sums with FMA, at the form's bar
+        eng.set_shape(L.FORM_FP64_FAST, 3, kt, 8, 0)
+        eng.run()
+        eng.store(s)
+        assert field_errors(s.gather(), ref, tt2).max() < 1e-12, f"FMA, tile of {kt}"
     eng.close()
     s.close()
     return ref, ran
