@@ -52,25 +52,28 @@ los_relayout_spline(const los_pair *pairs, const double *kc_all, const double *s
   const long base = pairs[p].src_off + (long)tp * ntau * n;
   const int lane = threadIdx.x;
 
-  // rows t0 .. t0+nt-1 of [tau][kc] are contiguous: nt * n doubles, read in
-  // batches of LOS_RS_B loads per lane so that they are all in flight at once
+  // rows t0 .. t0+nt-1 of [tau][kc]: 64/w rows of w lanes at a time (w: n rounded
+  // up to a power of two, at most 64), so that an element's row and column come
+  // from shifts; LOS_RS_B loads per lane are in flight at once
   {
     constexpr int LOS_RS_B = 32;
+    int sh = 6;
+    while (sh > 2 && (1 << (sh - 1)) >= n) --sh;
+    const int w = 1 << sh, rows = LOS_RS_TW >> sh, tr = lane >> sh;
     const double *r = raw + base + (long)t0 * n;
-    const int total = nt * n;
-    for (int i0 = 0; i0 < total; i0 += LOS_RS_TW * LOS_RS_B) {
-      double v[LOS_RS_B];
+    for (int c0 = 0; c0 < n; c0 += w) {
+      const int c = c0 + (lane & (w - 1));
+      for (int i0 = 0; i0 < nt; i0 += rows * LOS_RS_B) {
+        double v[LOS_RS_B];
 #pragma unroll
-      for (int u = 0; u < LOS_RS_B; ++u) {
-        const int i = i0 + u * LOS_RS_TW + lane;
-        v[u] = i < total ? r[i] : 0.0;
-      }
+        for (int u = 0; u < LOS_RS_B; ++u) {
+          const int t = i0 + u * rows + tr;
+          v[u] = t < nt && c < n ? r[t * n + c] : 0.0;
+        }
 #pragma unroll
-      for (int u = 0; u < LOS_RS_B; ++u) {
-        const int i = i0 + u * LOS_RS_TW + lane;
-        if (i < total) {
-          const int t = i / n;
-          tile[t * ls + (i - t * n)] = v[u];
+        for (int u = 0; u < LOS_RS_B; ++u) {
+          const int t = i0 + u * rows + tr;
+          if (t < nt && c < n) tile[t * ls + c] = v[u];
         }
       }
     }
@@ -83,10 +86,12 @@ los_relayout_spline(const los_pair *pairs, const double *kc_all, const double *s
   if (!cubic) return;
 
   if (live) {
-    const double *x = kc_all + pairs[p].kc_off;
-    const double *sig = spl + 3L * pairs[p].kc_off;
-    const double *pv = sig + n;
-    const double *gam = pv + n;
+    // the same for every lane and not written here: scalar loads
+    typedef const __attribute__((address_space(4))) double *uniform;
+    const uniform x = (uniform)(unsigned long long)(kc_all + pairs[p].kc_off);
+    const uniform sig = (uniform)(unsigned long long)(spl + 3L * pairs[p].kc_off);
+    const uniform pv = sig + n;
+    const uniform gam = pv + n;
     double *y = tile + lane * ls;  // y_i, then u_i, then the second derivatives
     const int a = n - 3, b = n - 2, e = n - 1;
     const double ya = y[a], yb = y[b], ye = y[e];
@@ -95,13 +100,16 @@ los_relayout_spline(const los_pair *pairs, const double *kc_all, const double *s
                 ((x[2] - x[0]) * (x[1] - x[0]) * (x[2] - x[1]));
     double u = (3.0 / (x[1] - x[0])) * ((y1 - y0) / (x[1] - x[0]) - d0);
     y[0] = u;
-    double ym = y0, yc = y1;
+    // sl: the slope over the interval to the left, the right one of the step before
+    double yc = y1, sl = (y1 - y0) / (x[1] - x[0]);
+#pragma unroll 4
     for (int i = 1; i < n - 1; ++i) {
       const double yn = y[i + 1];
-      double t = (yn - yc) / (x[i + 1] - x[i]) - (yc - ym) / (x[i] - x[i - 1]);
+      const double sr = (yn - yc) / (x[i + 1] - x[i]);
+      const double t = sr - sl;
       u = (6.0 * t / (x[i + 1] - x[i - 1]) - sig[i] * u) / pv[i];
       y[i] = u;
-      ym = yc;
+      sl = sr;
       yc = yn;
     }
     double dn = ((x[e] - x[a]) * (x[e] - x[a]) * (ye - yb) - (x[e] - x[b]) * (x[e] - x[b]) * (ye - ya)) /
@@ -110,6 +118,7 @@ los_relayout_spline(const los_pair *pairs, const double *kc_all, const double *s
     double un = (3.0 / (x[e] - x[b])) * (dn - (ye - yb) / (x[e] - x[b]));
     double next = (un - qn * u) / (qn * gam[n - 2] + 1.0);
     y[e] = next;
+#pragma unroll 4
     for (int k = n - 2; k >= 0; --k) {
       next = gam[k] * next + y[k];
       y[k] = next;
