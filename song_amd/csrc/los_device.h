@@ -62,8 +62,9 @@ typedef struct {
   const double *dd;     /* spline second derivatives, same layout */
   int F;                /* fine k3 total */
   /* Work order: n_pos positions, forder[s] the fine index at position s. The
-     positions of one job are contiguous and sorted by k3, so that workgroups
-     that run together on one XCD read neighbouring J rows and share its L2.
+     positions of one job (of all jobs together where tiles hold one position)
+     are contiguous and sorted by k3, so that workgroups that run together on one
+     XCD read neighbouring J rows and share its L2.
      Position s belongs to job pos_job[s] and writes column ocol[s] of it. */
   const int *forder;
   int n_pos;

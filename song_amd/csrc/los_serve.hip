@@ -158,6 +158,22 @@ static int launch_batch(los_server *S, slot_rec &sl, const std::vector<long> &id
     job_end.push_back((int)forder.size());
   }
   const int nk = S->shape.kind == 2 ? 64 : S->shape.nk;
+  if (S->shape.kind == 1 && nk == 1 && ids.size() > 1) {
+    // tiles of one position: the jobs' positions in one k3 order, so that waves that
+    // run together read neighbouring J rows whichever job they belong to
+    std::vector<int> by(forder.size());
+    for (size_t i = 0; i < by.size(); ++i) by[i] = (int)i;
+    std::stable_sort(by.begin(), by.end(),
+                     [&](int a, int b) { return e->hkf[forder[a]] < e->hkf[forder[b]]; });
+    const std::vector<int> f0 = forder, j0 = posjob, o0 = ocol;
+    const std::vector<double> c0 = cost;
+    for (size_t i = 0; i < by.size(); ++i) {
+      forder[i] = f0[by[i]];
+      posjob[i] = j0[by[i]];
+      ocol[i] = o0[by[i]];
+      cost[i] = c0[by[i]];
+    }
+  }
   std::vector<los_tile> tiles = make_tiles(job_end, nk);
 
   // descriptors, packed into one upload

@@ -13,6 +13,13 @@
 // (neighbouring k3 in the sorted work order). The reference's skip of rows
 // below index_xmin_J (source/transfer2.c:2232) is a select on the
 // interpolated J. No LDS and no barriers: waves are independent.
+//
+// Bound by the J rows it fetches. Two things keep a wave from fetching what it
+// need not: a lane none of whose rows lives at the element's index_x is given an
+// offset out of the table (64 l span a wide range of first live points), and the
+// row registers outlive the step (index_x stays for several early steps). Plain
+// FP64, tiles of one k3: 3,098 k3 x 251 steps x 37 l x m = 0, 2: 1.87 to 1.18 ms;
+// 14,753 k3 x 600 steps x 96 l x m = 0, 1, 2: 61.4 to 42.4 ms.
 #pragma once
 
 #include <hip/hip_runtime.h>
@@ -41,6 +48,9 @@ template <class R>
 struct alignas(2 * sizeof(R)) SweepPair {
   R j0, j1;
 };
+
+// A lane offset beyond any table (LOS_BUF_MAX): the load touches no memory.
+#define SWEEP_OUT 0xFFFFFF00u
 
 // The J table is read through a raw buffer resource: a load adds the lane's
 // byte offset (lane slot) to a wave-uniform 32-bit byte offset (row and x), so
@@ -508,6 +518,11 @@ __device__ __forceinline__ void sweep_item(const los_params &P, int xcd, int q, 
   int fl = f[0];  // this lane's element (lanes below NK)
 #pragma unroll
   for (int j = 1; j < NK; ++j) fl = li == j ? f[j] : fl;
+  // a lane whose rows are all dead at the element's index_x reads nothing (an
+  // offset out of the resource's range gives 0); `held` is the index_x in the row
+  // registers, which outlives the step
+  const int xml = active ? P.min_xmin[lm] : INT_MAX;
+  int held = -1;
   SweepIXA<R> nxt{};
   if (li < NK && tend > 0) nxt = ixa[(long)fl * P.ntau];
 
@@ -534,15 +549,16 @@ __device__ __forceinline__ void sweep_item(const los_params &P, int xcd, int q, 
       // usually share it), so one set of row registers serves the tile
 #pragma unroll
       for (int j = 0; j < NK; ++j) {
-        if (j == 0 || ix[j] != ix[j - 1]) {
-          const unsigned ox = (unsigned)ix[j] * xstep;
+        if (ix[j] != held) {
+          held = ix[j];
+          const unsigned ox = (unsigned)ix[j] * xstep, lo = held >= xml ? lane : SWEEP_OUT;
 #pragma unroll
           for (int L = 0; L < NL; ++L) {
             if (m > L) continue;
-            if (doT && L <= P.LmaxT) tv[L] = sweep_load<R, PAIRS>(Jr, lane, bT + L * rowb + ox, xstep);
+            if (doT && L <= P.LmaxT) tv[L] = sweep_load<R, PAIRS>(Jr, lo, bT + L * rowb + ox, xstep);
             if (doP && L <= P.LmaxP) {
-              ev[L] = sweep_load<R, PAIRS>(Jr, lane, bE + L * rowb + ox, xstep);
-              if (mix) qv[L] = sweep_load<R, PAIRS>(Jr, lane, bQ + L * rowb + ox, xstep);
+              ev[L] = sweep_load<R, PAIRS>(Jr, lo, bE + L * rowb + ox, xstep);
+              if (mix) qv[L] = sweep_load<R, PAIRS>(Jr, lo, bQ + L * rowb + ox, xstep);
             }
           }
         }
@@ -786,6 +802,11 @@ __device__ __forceinline__ void sweep_exact_item(const los_params &P, int xcd, i
   int fl = f[0];  // this lane's element (lanes below NK)
 #pragma unroll
   for (int j = 1; j < NK; ++j) fl = li == j ? f[j] : fl;
+  // a lane whose rows are all dead at the element's index_x reads nothing (an
+  // offset out of the resource's range gives 0, as the table does there); `held` is
+  // the index_x in the row registers, which outlives the step
+  const int xml = active ? P.min_xmin[lm] : INT_MAX;
+  int held = -1;
   SweepIXA<double> nxt{0, 0, 0.};
   if (li < NK && tend > 0) nxt = ixa[(long)fl * P.ntau];
   for (int t = 0; t < tend; ++t) {
@@ -804,21 +825,22 @@ __device__ __forceinline__ void sweep_exact_item(const los_params &P, int xcd, i
       src[j] = li < 3 * NL ? sf[(((long)f[j] * P.ntau + t) * P.m_size + mi) * 3 * NL + li] : 0.;
 #pragma unroll
     for (int j = 0; j < NK; ++j) {
-      if (j == 0 || ix[j] != ix[j - 1]) {
-        const unsigned ox = (unsigned)ix[j] * xstep;
+      if (ix[j] != held) {
+        held = ix[j];
+        const unsigned ox = (unsigned)ix[j] * xstep, lo = held >= xml ? lane : SWEEP_OUT;
 #pragma unroll
         for (int L = 0; L < NL; ++L) {
           if (m > L) continue;
           if (doT && L <= P.LmaxT) {
-            tv[L] = sweep_row<double>(Jr, lane, bT + L * rowb + ox, xstep);
-            if (CUBIC) td[CUBIC ? L : 0] = sweep_row<double>(Dr, lane, bT + L * rowb + ox, xstep);
+            tv[L] = sweep_row<double>(Jr, lo, bT + L * rowb + ox, xstep);
+            if (CUBIC) td[CUBIC ? L : 0] = sweep_row<double>(Dr, lo, bT + L * rowb + ox, xstep);
           }
           if (doP && L <= P.LmaxP) {
-            ev[L] = sweep_row<double>(Jr, lane, bE + L * rowb + ox, xstep);
-            qv[L] = sweep_row<double>(Jr, lane, bQ + L * rowb + ox, xstep);
+            ev[L] = sweep_row<double>(Jr, lo, bE + L * rowb + ox, xstep);
+            qv[L] = sweep_row<double>(Jr, lo, bQ + L * rowb + ox, xstep);
             if (CUBIC) {
-              ed[CUBIC ? L : 0] = sweep_row<double>(Dr, lane, bE + L * rowb + ox, xstep);
-              qd[CUBIC ? L : 0] = sweep_row<double>(Dr, lane, bQ + L * rowb + ox, xstep);
+              ed[CUBIC ? L : 0] = sweep_row<double>(Dr, lo, bE + L * rowb + ox, xstep);
+              qd[CUBIC ? L : 0] = sweep_row<double>(Dr, lo, bQ + L * rowb + ox, xstep);
             }
           }
         }
