@@ -18,11 +18,15 @@
 // pair's two triangle-edge points (the first point with k3 >= k1 - k2 before
 // the last, and the first point after the first whose successor lies beyond
 // k1 + k2, the point past the end counting as beyond) are resolved once, so
-// every k3 term is independent: los_cl2_partial runs CL2_CHUNKS workgroups of
-// 256 threads per (l, m) row over the flat k3 index and reduces in LDS in a
-// fixed order; los_cl2_finish adds a row's chunk sums in order. Results are
-// deterministic; the sum order differs from the reference's sequential one,
-// so they agree to rounding (relative 1e-12 of the sum of |terms|).
+// every k3 term is independent: los_cl2_weights makes the terms without the
+// transfers once per m, los_cl2_partial runs up to CL2_CHUNKS workgroups of 256
+// threads per (l, m) row over the flat k3 index and reduces in a fixed order, and
+// los_cl2_finish adds a row's chunk sums in order (a row of one chunk, up to 4096
+// points, makes its terms itself and needs no other kernel). Results are
+// deterministic; the sum order differs from the reference's sequential one, so
+// they agree to rounding (relative 1e-12 of the sum of |terms|).
+// 96 l, m = 0, 1, 2, 17,700 k3 points: 27 us in three launches (4.5 + 16.5 + 3.9, the
+// transfers 82 MB at 5 TB/s), 38 us with each row making its own terms in 32 chunks.
 #include <hip/hip_runtime.h>
 
 #include <cmath>
@@ -46,7 +50,14 @@
     }                                                                                        \
   } while (0)
 
-#define CL2_CHUNKS 32
+#define CL2_CHUNKS 32 /* most parts of a row */
+
+// Parts of a row: 4096 terms (16 a thread) each; one part needs no second kernel.
+static int cl2_chunks(long n_k3)
+{
+  const long c = (n_k3 + 4095) / 4096;
+  return (int)(c < 1 ? 1 : c > CL2_CHUNKS ? CL2_CHUNKS : c);
+}
 
 struct los_cl2 {
   int device;
@@ -56,6 +67,7 @@ struct los_cl2 {
   hipStream_t stream;
   hipEvent_t ev0, ev1;
   double *k3, *t1, *t2, *out, *partial, *pq;  // pq: per pair k1 k2 s1 s2 sp1 sp2
+  double *weight;                              // per m and k3, where rows have several parts
   long *pair_off;
   int *pair_of, *edge, *m, *used;             // edge: per pair first, last
 };
@@ -82,60 +94,95 @@ __device__ __forceinline__ double cl2_factor(double k1, double k2, double k3, do
          M_PI * sp1 * sp2;
 }
 
+// Term i (of n_k3) without the transfers; -0. where the reference skips it (no
+// half step).
+__device__ __forceinline__ double cl2_term(const long *__restrict__ pair_off,
+                                           const int *__restrict__ pair_of,
+                                           const int *__restrict__ edge,
+                                           const double *__restrict__ pq,
+                                           const double *__restrict__ k3g, long i, int m,
+                                           int rescale)
+{
+  const int p = pair_of[i];
+  const long b = pair_off[p];
+  const int n = (int)(pair_off[p + 1] - b);
+  const int j = (int)(i - b);
+  const double *g = k3g + b;
+  const double *q = pq + 6 * (long)p;
+  const double k1 = q[0], k2 = q[1];
+  const double k3 = g[j];
+  double s3;
+  // half trapezoid step and triangle-edge corrections (:486-500)
+  if (j == edge[2 * p + 1]) s3 = (k3 - g[j - 1]) / 2. + (k1 + k2) - k3;
+  else if (j == edge[2 * p]) s3 = (g[j + 1] - k3) / 2. + k3 - (k1 - k2);
+  else if (k3 < k1 - k2 || k3 > k1 + k2) s3 = 0.;
+  else if (j == 0) s3 = (g[1] - g[0]) / 2.;
+  else if (j == n - 1) s3 = (g[n - 1] - g[n - 2]) / 2.;
+  else s3 = (g[j + 1] - g[j - 1]) / 2.;
+  if (s3 == 0) return -0.;
+  return cl2_factor(k1, k2, k3, q[2], q[3], s3, q[4], q[5], m, rescale);
+}
+
+// Every term of every m once, weight[m][i]: the rows of all l share them (some 20
+// divisions a term).
+__global__ void __launch_bounds__(CL2_THREADS)
+los_cl2_weights(const long *__restrict__ pair_off, const int *__restrict__ pair_of,
+                const int *__restrict__ edge, const double *__restrict__ pq,
+                const double *__restrict__ k3g, long n_k3, const int *__restrict__ mv, int m_size,
+                int rescale, double *__restrict__ weight)
+{
+  const long n = n_k3 * m_size, e = (long)blockIdx.x * CL2_THREADS + threadIdx.x;
+  if (e >= n) return;
+  const int im = (int)(e / n_k3);
+  weight[e] = cl2_term(pair_off, pair_of, edge, pq, k3g, e - im * n_k3, mv[im], rescale);
+}
+
+// Sums of `chunks` interleaved parts of a row's terms. WEIGHTS: the terms from
+// los_cl2_weights; otherwise made here, with the same operations.
+template <bool WEIGHTS>
 __global__ void __launch_bounds__(CL2_THREADS)
 los_cl2_partial(const long *__restrict__ pair_off, const int *__restrict__ pair_of,
                 const int *__restrict__ edge, const double *__restrict__ pq,
                 const double *__restrict__ k3g, long n_k3, const double *__restrict__ t1,
                 const double *__restrict__ t2, const int *__restrict__ mv, int m_size,
-                const int *__restrict__ used, int rescale, double *__restrict__ partial)
+                const int *__restrict__ used, int rescale, int chunks,
+                const double *__restrict__ weight, double *__restrict__ partial)
 {
-  __shared__ double part[CL2_THREADS];
-  const int chunk = blockIdx.x % CL2_CHUNKS;
-  const long row = blockIdx.x / CL2_CHUNKS;
-  const int m = mv[row % m_size];
+  __shared__ double part[CL2_THREADS / 64];
+  const long row = blockIdx.x / chunks;
+  const int chunk = (int)(blockIdx.x - row * chunks);
+  const int im = (int)(row % m_size), m = mv[im];
   double acc = 0.;
   if (used[row]) {
     const double *T1 = t1 + row * n_k3;
     const double *T2 = t2 + row * n_k3;
+    const double *W = WEIGHTS ? weight + im * n_k3 : nullptr;
+#pragma unroll 4
     for (long i = (long)chunk * CL2_THREADS + threadIdx.x; i < n_k3;
-         i += (long)CL2_CHUNKS * CL2_THREADS) {
-      const int p = pair_of[i];
-      const long b = pair_off[p];
-      const int n = (int)(pair_off[p + 1] - b);
-      const int j = (int)(i - b);
-      const double *g = k3g + b;
-      const double *q = pq + 6 * (long)p;
-      const double k1 = q[0], k2 = q[1];
-      const double k3 = g[j];
-      double s3;
-      // half trapezoid step and triangle-edge corrections (:486-500)
-      if (j == edge[2 * p + 1]) s3 = (k3 - g[j - 1]) / 2. + (k1 + k2) - k3;
-      else if (j == edge[2 * p]) s3 = (g[j + 1] - k3) / 2. + k3 - (k1 - k2);
-      else if (k3 < k1 - k2 || k3 > k1 + k2) s3 = 0.;
-      else if (j == 0) s3 = (g[1] - g[0]) / 2.;
-      else if (j == n - 1) s3 = (g[n - 1] - g[n - 2]) / 2.;
-      else s3 = (g[j + 1] - g[j - 1]) / 2.;
-      if (s3 == 0) continue;
-      const double f = cl2_factor(k1, k2, k3, q[2], q[3], s3, q[4], q[5], m, rescale);
-      acc += f * T1[i] * T2[i];
+         i += (long)chunks * CL2_THREADS) {
+      const double f = WEIGHTS ? W[i] : cl2_term(pair_off, pair_of, edge, pq, k3g, i, m, rescale);
+      const double v = f * T1[i] * T2[i];
+      acc = f == 0. && __builtin_signbit(f) ? acc : acc + v;
     }
   }
-  part[threadIdx.x] = acc;
+  for (int w = 32; w > 0; w >>= 1) acc += __shfl_xor(acc, w);
+  if ((threadIdx.x & 63) == 0) part[threadIdx.x >> 6] = acc;
   __syncthreads();
-  for (int w = CL2_THREADS / 2; w > 0; w >>= 1) {
-    if (threadIdx.x < w) part[threadIdx.x] += part[threadIdx.x + w];
-    __syncthreads();
+  if (threadIdx.x == 0) {
+    double v = part[0];
+    for (int w = 1; w < CL2_THREADS / 64; ++w) v += part[w];
+    partial[row * chunks + chunk] = v;
   }
-  if (threadIdx.x == 0) partial[row * CL2_CHUNKS + chunk] = part[0];
 }
 
 __global__ void __launch_bounds__(64)
-los_cl2_finish(const double *__restrict__ partial, long rows, double *__restrict__ out)
+los_cl2_finish(const double *__restrict__ partial, long rows, int chunks,
+               double *__restrict__ out)
 {
   const long row = (long)blockIdx.x * 64 + threadIdx.x;
   if (row >= rows) return;
   double v = 0.;
-  for (int c = 0; c < CL2_CHUNKS; ++c) v += partial[row * CL2_CHUNKS + c];
+  for (int c = 0; c < chunks; ++c) v += partial[row * chunks + c];
   out[row] = v;
 }
 
@@ -153,7 +200,7 @@ void los_cl2_destroy(los_cl2 *h)
 {
   if (!h) return;
   hipSetDevice(h->device);
-  void *bufs[] = {h->k3, h->t1, h->t2, h->out, h->partial, h->pq,
+  void *bufs[] = {h->k3, h->t1, h->t2, h->out, h->partial, h->pq, h->weight,
                   h->pair_off, h->pair_of, h->edge, h->m, h->used};
   for (void *b : bufs)
     if (b) hipFree(b);
@@ -246,6 +293,8 @@ int los_cl2_create(const los_cl2_desc *d, int device, los_cl2 **out, char *errms
   if (e == hipSuccess) e = hipMalloc((void **)&h->out, (size_t)(rows > 0 ? rows : 1) * 8);
   if (e == hipSuccess)
     e = hipMalloc((void **)&h->partial, (size_t)(rows > 0 ? rows : 1) * CL2_CHUNKS * 8);
+  if (e == hipSuccess && cl2_chunks(n_k3) > 1)
+    e = hipMalloc((void **)&h->weight, (size_t)n_k3 * d->m_size * 8);
   if (e != hipSuccess) {
     snprintf(errmsg, _ERRORMSGSIZE_, "los_cl2_create: %s", hipGetErrorString(e));
     los_cl2_destroy(h);
@@ -264,12 +313,25 @@ int los_cl2_run(los_cl2 *h, int reps, float *ms, char *errmsg)
   if (reps < 1) reps = 1;
   CCHK(hipEventRecord(h->ev0, h->stream));
   los_test(rows * CL2_CHUNKS > 0x7fffffffL, errmsg, "los_cl2_run: too many rows");
+  const int chunks = cl2_chunks(h->n_k3);
+  const long terms = h->n_k3 * h->m_size;
   for (int i = 0; i < reps; ++i) {
-    hipLaunchKernelGGL(los_cl2_partial, dim3((unsigned)(rows * CL2_CHUNKS)), dim3(CL2_THREADS),
+    if (chunks == 1) {
+      hipLaunchKernelGGL(los_cl2_partial<false>, dim3((unsigned)rows), dim3(CL2_THREADS), 0,
+                         h->stream, h->pair_off, h->pair_of, h->edge, h->pq, h->k3, h->n_k3, h->t1,
+                         h->t2, h->m, h->m_size, h->used, h->rescale, 1, (const double *)nullptr,
+                         h->out);
+      continue;
+    }
+    hipLaunchKernelGGL(los_cl2_weights, dim3((unsigned)((terms + CL2_THREADS - 1) / CL2_THREADS)),
+                       dim3(CL2_THREADS), 0, h->stream, h->pair_off, h->pair_of, h->edge, h->pq,
+                       h->k3, h->n_k3, h->m, h->m_size, h->rescale, h->weight);
+    hipLaunchKernelGGL(los_cl2_partial<true>, dim3((unsigned)(rows * chunks)), dim3(CL2_THREADS),
                        0, h->stream, h->pair_off, h->pair_of, h->edge, h->pq, h->k3, h->n_k3,
-                       h->t1, h->t2, h->m, h->m_size, h->used, h->rescale, h->partial);
+                       h->t1, h->t2, h->m, h->m_size, h->used, h->rescale, chunks, h->weight,
+                       h->partial);
     hipLaunchKernelGGL(los_cl2_finish, dim3((unsigned)((rows + 63) / 64)), dim3(64), 0,
-                       h->stream, h->partial, rows, h->out);
+                       h->stream, h->partial, rows, chunks, h->out);
   }
   CCHK(hipGetLastError());
   CCHK(hipEventRecord(h->ev1, h->stream));
@@ -394,11 +456,14 @@ extern "C" int los_cl2_sum_noalloc(const los_cl2_desc *d, long n_k3, double *cl_
   const int n_pairs = d->k_size * (d->k_size + 1) / 2;
   hipLaunchKernelGGL(los_cl2_pairs, dim3((n_pairs + 63) / 64), dim3(64), 0, s, d->k_size, d->k,
                      d->pk, d->pair_off, d->k3, pq, edge, pair_of);
-  hipLaunchKernelGGL(los_cl2_partial, dim3((unsigned)(rows * CL2_CHUNKS)), dim3(CL2_THREADS), 0,
+  const int chunks = cl2_chunks(n_k3);
+  hipLaunchKernelGGL(los_cl2_partial<false>, dim3((unsigned)(rows * chunks)), dim3(CL2_THREADS), 0,
                      s, d->pair_off, pair_of, edge, pq, d->k3, n_k3, d->transfer1, d->transfer2,
-                     d->m, d->m_size, d->used, d->rescale, partial);
-  hipLaunchKernelGGL(los_cl2_finish, dim3((unsigned)((rows + 63) / 64)), dim3(64), 0, s, partial,
-                     rows, cl_m);
+                     d->m, d->m_size, d->used, d->rescale, chunks, (const double *)nullptr,
+                     chunks == 1 ? cl_m : partial);
+  if (chunks > 1)
+    hipLaunchKernelGGL(los_cl2_finish, dim3((unsigned)((rows + 63) / 64)), dim3(64), 0, s, partial,
+                       rows, chunks, cl_m);
   CCHK(hipGetLastError());
   return _SUCCESS_;
 }
