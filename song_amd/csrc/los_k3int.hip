@@ -56,6 +56,28 @@ struct los_k3int {
   double alg_bytes;
 };
 
+typedef double k3_d2 __attribute__((ext_vector_type(2), aligned(8)));
+
+// y / step as IEEE division gives it. FAST: with r = 1/step rounded to nearest, one
+// Newton correction makes q faithful and a second one correctly rounded (Markstein's
+// theorem), where step is far from the ends of the exponent range (the host checks)
+// and so is the remainder; the quotients here are at most the table's size, and where
+// y is too small for an exact remainder only (int)q = 0 is used.
+template <bool FAST>
+__device__ __forceinline__ double k3_div(double y, double step, double r)
+{
+  if (!FAST) return y / step;
+  double q = y * r;
+  q = __builtin_fma(__builtin_fma(-q, step, y), r, q);
+  return __builtin_fma(__builtin_fma(-q, step, y), r, q);
+}
+
+// Bound by the FP64 instructions of a term and the gathers of its two nodes: 48 l3
+// rows, 136 pairs, 100 r (11,178 k3), 185 us; with two IEEE divisions a term
+// (about ten instructions each), one term at a time, 264 us.
+// Four terms at a time: their values come with scalar loads, and the j nodes of all
+// four are in flight together. A wave skips four terms that none of its lanes wants.
+template <bool FAST>
 __global__ void __launch_bounds__(64)
 los_k3int_kernel(const long *__restrict__ pair_off, const double *__restrict__ k3,
                  const double *__restrict__ dk3, const double *__restrict__ transfer, long n_k3,
@@ -64,6 +86,7 @@ los_k3int_kernel(const long *__restrict__ pair_off, const double *__restrict__ k
                  const double *__restrict__ rr, int n_r, int n_pairs, int n_rc, double coef,
                  double *__restrict__ out)
 {
+  constexpr int U = 4;
   const int rc = blockIdx.x % n_rc;
   const int p = (blockIdx.x / n_rc) % n_pairs;
   const int q = blockIdx.x / (n_rc * n_pairs);
@@ -72,22 +95,42 @@ los_k3int_kernel(const long *__restrict__ pair_off, const double *__restrict__ k
   const int iL = index_L[q];
   double integral = 0.0;
   if (iL >= 0) {
-    const double r = rr[ir];
+    const double r = rr[ir], rstep = 1. / step;
     const double xmin = x_min[iL];
     const double *J = jtab + j_off[iL];
     const double *T = transfer + (long)q * n_k3;
     const long b = pair_off[p], e = pair_off[p + 1];
-    for (long i = b; i < e; ++i) {
-      const double f = T[i];
-      if (f == 0.) continue;
-      const double k = k3[i];
-      const double x = k * r;
-      if (x < xmin) continue;
-      const int ix = (int)((x - xmin) / step);
-      const double a = (xmin + step * (ix + 1) - x) / step;
-      const double jv = a * J[ix] + (1. - a) * J[ix + 1];
-      const double integrand = k * k * jv * f;
-      integral += integrand * dk3[i];
+    for (long i0 = b; i0 < e; i0 += U) {
+      double x[U], f[U], k[U], d[U];
+      bool in[U], any = false;
+#pragma unroll
+      for (int u = 0; u < U; ++u) {
+        const long i = min(i0 + u, e - 1);
+        f[u] = T[i];
+        k[u] = k3[i];
+        d[u] = dk3[i];
+      }
+#pragma unroll
+      for (int u = 0; u < U; ++u) {
+        x[u] = k[u] * r;
+        in[u] = i0 + u < e && f[u] != 0. && !(x[u] < xmin);
+        any |= in[u];
+      }
+      if (__ballot(any) == 0) continue;
+      double a[U];
+      k3_d2 j[U];
+#pragma unroll
+      for (int u = 0; u < U; ++u) {
+        const int ix = in[u] ? (int)k3_div<FAST>(x[u] - xmin, step, rstep) : 0;
+        a[u] = k3_div<FAST>(xmin + step * (ix + 1) - x[u], step, rstep);
+        j[u] = *(const k3_d2 *)(J + ix);
+      }
+#pragma unroll
+      for (int u = 0; u < U; ++u) {
+        const double jv = a[u] * j[u].x + (1. - a[u]) * j[u].y;
+        const double integrand = k[u] * k[u] * jv * f[u];
+        integral = in[u] ? integral + integrand * d[u] : integral;
+      }
     }
     integral *= 0.5;
     integral *= coef;
@@ -243,8 +286,10 @@ int los_k3int_run(los_k3int *h, int reps, float *ms, char *errmsg)
   los_test(blocks > 0x7fffffffL, errmsg, "los_k3int_run: %ld workgroups is too many", blocks);
   if (reps < 1) reps = 1;
   KCHK(hipEventRecord(h->ev0, h->stream));
+  const auto kernel = h->xx_step > 1e-100 && h->xx_step < 1e100 ? los_k3int_kernel<true>
+                                                                : los_k3int_kernel<false>;
   for (int i = 0; i < reps; ++i)
-    hipLaunchKernelGGL(los_k3int_kernel, dim3((unsigned)blocks), dim3(64), 0, h->stream,
+    hipLaunchKernelGGL(kernel, dim3((unsigned)blocks), dim3(64), 0, h->stream,
                        h->pair_off, h->k3, h->dk3, h->transfer, h->n_k3, h->index_L, h->j_off,
                        h->j, h->x_min, h->xx_step, h->r, h->n_r, h->n_pairs, n_rc, h->coef,
                        h->out);
