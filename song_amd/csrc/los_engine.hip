@@ -1140,10 +1140,34 @@ int ensure_klane(los_engine *e, const los_shape *sh, char *err)
 }
 
 // Device tables a window shape needs (allocated outside any capture).
+// Frees the per-(k3, tau) tables of a kernel kind (made again when a shape of it
+// is chosen), so that tuning holds those of one kind at a time.
+static void release_tables(los_engine *e, int kind)
+{
+  auto drop = [](void *&p) {
+    if (p) (void)hipFree(p);
+    p = nullptr;
+  };
+  if (kind == 1) {
+    drop(e->dixa);
+    drop(e->dsf);
+    e->sweep_form = -1;
+  } else if (kind == 2) {
+    drop(e->dkixa);
+    drop(e->dksrc);
+    e->klane_form = -1;
+  } else if (kind == 3) {
+    dfree(e->dwix);
+    dfree(e->dwaj);
+    dfree(e->dwsrc);
+  }
+}
+
 static int ensure_window(los_engine *e, const los_shape *sh, char *err)
 {
   if (sh == nullptr || sh->kind != 3) return _SUCCESS_;
   if (e->dwsrc) return _SUCCESS_;
+  release_tables(e, 3);  // what a failed allocation left
   const size_t n = (size_t)e->P.k_npad * e->ntau;
   size_t rows = 0;
   for (int set = 0; set < 2; ++set)
@@ -1234,7 +1258,9 @@ extern "C" int los_engine_autotune(los_engine *e, int reps, char *err)
   }
   float best = 1e30f;
   int ibest = 0;
+  drop_graph(e);  // it reads tables that are freed below
   for (int i = 0; i < nc; ++i) {
+    if (i > 0 && cand[i].kind != cand[i - 1].kind) release_tables(e, cand[i - 1].kind);
     // each shape timed on whole steps: its own preparation and tables, then its kernel
     if (ensure_tables(e, &cand[i], err)) return _FAILURE_;
     if (enqueue_prep(e, &cand[i], err) || enqueue_los(e, &cand[i], err))  // warm-up
@@ -1251,9 +1277,10 @@ extern "C" int los_engine_autotune(los_engine *e, int reps, char *err)
       ibest = i;
     }
   }
+  for (int kind = 1; kind <= 3; ++kind)
+    if (kind != cand[ibest].kind) release_tables(e, kind);
   e->shape[form] = cand[ibest];
   e->shape_set[form] = true;
-  drop_graph(e);
   std::lock_guard<std::mutex> g(g_tuned_mu);
   g_tuned[key] = cand[ibest];
   return _SUCCESS_;

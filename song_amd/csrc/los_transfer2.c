@@ -815,8 +815,10 @@ int los_server_create(int device, int form, double hbm_budget_bytes, int n_slots
 
 /* Device bytes of one k1 batch's pairs beyond the resident J tables: the
    sources three times (as SONG lays them out, re-laid out, spline second
-   derivatives), and per fine k3 the outputs, the per-(k3, tau) tables of the
-   sweep and k-lane kernels (the autotuner may build both) and small lists.
+   derivatives), and per fine k3 the outputs, the per-(k3, tau) tables and small
+   lists. The tables are counted as those of the sweep and the k-lane kernels
+   together; the autotuner holds those of one kind at a time, and the window
+   kernels' are no larger than the sweep kernels'.
    SONG_LOS_BATCH_BYTES in the environment replaces the budget (bytes), so that
    smaller batches can be asked for. */
 static double batch_bytes(const los_stage *st, int k1_begin, int k1_end)
