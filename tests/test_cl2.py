@@ -192,3 +192,30 @@ def test_cl2_on_gpu_transfers():
     s.close()
     assert np.all(ref > 0)
     assert np.allclose(got, ref, rtol=1e-12, atol=0)
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("n_k3", [6, 4095, 4096, 4097, 131072, 131073])
+def test_cl2_parts_of_a_row(n_k3):
+    """One part, one more than a part, all 32 and uneven ones; unused rows among them."""
+    print(f"case cl2 n_k3={n_k3}", flush=True)
+    rng = np.random.default_rng(n_k3)
+    k = np.geomspace(1e-3, 0.1, 2 if n_k3 < 20 else 4)
+    n = np.full(k.size * (k.size + 1) // 2, n_k3 // (k.size * (k.size + 1) // 2))
+    n[-1] += n_k3 - n.sum()
+    pairs = [(a, b) for i, a in enumerate(k) for b in k[:i + 1]]
+    k3 = np.concatenate([np.linspace(a - b + 0.01 * b, a + b - 0.01 * b, c)
+                         for (a, b), c in zip(pairs, n)])
+    po = np.concatenate([[0], np.cumsum(n)])
+    assert k3.size == n_k3 and po[-1] == n_k3
+    pk = 2.1e-9 * (k / 0.05) ** (0.965 - 1)
+    t1, t2 = rng.standard_normal((2, 3, 2, n_k3))
+    used = np.array([[1, 1], [0, 1], [1, 1]], dtype=np.int32)
+    _, ref = oracle_cl2(k, pk, po, k3, [0, 2], t1, t2, used, 1)
+    _, scale = oracle_cl2(k, pk, po, k3, [0, 2], np.abs(t1), np.abs(t2), used, 1)
+    h = L.Cl2(k, pk, po, k3, [0, 2], t1, t2, used, 1)
+    h.run(2)
+    got = h.result()
+    h.close()
+    assert got[1, 0] == 0
+    assert np.all(np.abs(got - ref) <= 1e-12 * scale)

@@ -197,3 +197,26 @@ def test_k3int_on_gpu_transfers(oracle):
     s.close()
     assert np.count_nonzero(ref) > 0.5 * ref.size
     assert np.array_equal(got, ref)
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("n_k3", [2, 3, 4, 5, 7, 8, 9])
+@pytest.mark.parametrize("step", [0.3, 0.25, 1e101])
+def test_k3int_remainders_and_steps(n_k3, step):
+    """Counts about the terms a lane holds in flight; a step outside the range in which its
+    reciprocal replaces the division."""
+    print(f"case k3int n_k3={n_k3} step={step}", flush=True)
+    rng = np.random.default_rng(n_k3)
+    pair_off = np.array([0, n_k3, 2 * n_k3])
+    k3 = np.sort(rng.uniform(1e-4, 0.2, (2, n_k3)), axis=1).ravel()
+    n_x = 100 if step > 1e100 else int(0.2 * 900 / step) + 4
+    j_off, j = np.array([0, n_x]), rng.standard_normal(n_x)
+    args = (pair_off, k3, rng.standard_normal((1, k3.size)), [0], j_off, j, [0.0], step,
+            np.linspace(1.0, 900.0, 70))
+    ref = oracle_k3int(*args, 0, 1.0)
+    h = L.K3Integral(*args, 1.0)
+    h.run(1)
+    got = h.result()
+    h.close()
+    assert np.count_nonzero(ref) > 0.5 * ref.size
+    assert np.array_equal(got, ref)
