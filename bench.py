@@ -103,11 +103,11 @@ def kernel_name(form: str, shape, nl: int) -> str:
     kind, nk, ch, pers = shape
     flag = "true" if pers else "false"
     if form == "fp64":
-        return (f"los_window<false, {nl}, {ch}, {64 // nk}>" if kind == 3 else
+        return (f"los_window<0, {nl}, {ch}, {64 // nk}>" if kind == 3 else
                 f"los_sweep_exact<{nk}, {nl}, {flag}>" if kind == 1 else
                 f"los_klane_exact<{nl}, {ch}>" if kind == 2 else f"los_integrate_exact<{nl}>")
     if kind == 3:
-        return f"los_window<true, {nl}, {ch}, {64 // nk}>"
+        return f"los_window<{1 if form == 'fp64fast' else 2}, {nl}, {ch}, {64 // nk}>"
     pol = POLICY[form]
     if kind == 1:
         pairs = "true" if (form == "fp64fast" or ch == 1) else "false"

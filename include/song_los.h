@@ -117,8 +117,8 @@ int los_engine_last_kernel_ms(los_engine *eng, float *ms_los, float *ms_spline);
    kind 1, the sweep, and kind 2, the k-lane kernel below; kind 3, the "window"
    kernel: one wave per (nk = 64, 32 or 16 neighbouring fine k3, m, T or E and B,
    ch = 8 l, 4 with B sources) with the J rows' windows in LDS, offered where the
-   batch's k3 lie close enough. All keep the reference's operations. The FMA-FP64
-   form has kind 3 as well.
+   batch's k3 lie close enough. All keep the reference's operations. The fast
+   forms have kind 3 as well.
    Fast forms: kind 0, the "stream" kernel: nk fine k3 per workgroup, ch time
    steps per LDS chunk, persistent = 1 for the chip-sized grid fed by the device
    work queue; kind 1, the "sweep" kernel: one wave per (nk fine k3, m, 64 l)

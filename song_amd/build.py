@@ -27,6 +27,7 @@ HIP_SOURCES = [
     ("los_kernels_exact.hip", ["-ffp-contract=off"]),
     ("los_kernels_window.hip", ["-ffp-contract=off"]),
     ("los_kernels_window_fma.hip", []),
+    ("los_kernels_window_f32.hip", []),
     ("los_kernels_fast.hip", []),
     ("los_serve.hip", []),
     ("los_bessel2_gpu.hip", ["-ffp-contract=off"]),

@@ -931,9 +931,8 @@ static int form_shapes(const los_engine *e, int form, los_shape *out, int cap)
   } else {
     n = los_shapes(form == LOS_FORM_FP32C, e->loaded ? e->P.tp2_size : 1, all, 48);
   }
-  if (form != LOS_FORM_FP32C)
-    for (int kt = 64; kt >= 16; kt /= 2)
-      if (window_fits(e, kt)) all[n++] = los_shape{3, kt, 8, 0};
+  for (int kt = 64; kt >= 16; kt /= 2)
+    if (window_fits(e, kt)) all[n++] = los_shape{3, kt, 8, 0};
   int k = 0;
   for (int i = 0; i < n && k < cap; ++i) {
     // cubic interpolation of J: the plain FP64 sweep kernels only
@@ -972,8 +971,8 @@ int enqueue_los_params(los_engine *e, const los_shape *sh, los_params *P, hipStr
   if (sh->kind == 3) {
     // sh->ch = 8 (l,m) offsets a wave, 4 where it holds the rows of two J types
     const int slot = nk_slot(sh->nk), gs[2] = {P->has_B ? 2 : 3, 3};
-    P->Jk = e->dJk;
-    P->Jk_bytes = (unsigned)(e->nJk * sizeof(double));
+    P->Jk = fp32 ? (const void *)e->dJk32 : (const void *)e->dJk;
+    P->Jk_bytes = (unsigned)(e->nJk * (fp32 ? sizeof(float) : sizeof(double)));
     for (int set = 0; set < 2; ++set) {
       P->wgrp[set] = e->dkgrp[gs[set]];
       for (int im = 0; im <= LOS_MAX_MI; ++im)
@@ -985,6 +984,8 @@ int enqueue_los_params(los_engine *e, const los_shape *sh, los_params *P, hipStr
     std::copy(e->wxcd[slot], e->wxcd[slot] + 9, P->xcd_tile);
     if (e->form == LOS_FORM_FP64)
       HIPCHK(los_launch_window_exact(P, sh->nk, sh->ch, s), err);
+    else if (fp32)
+      HIPCHK(los_launch_window_f32(P, sh->nk, sh->ch, s), err);
     else
       HIPCHK(los_launch_window_fma(P, sh->nk, sh->ch, s), err);
     return _SUCCESS_;
@@ -1053,7 +1054,10 @@ static int enqueue_tables(los_engine *e, const los_shape *sh, char *err, int f_b
     else
       HIPCHK(los_launch_klane_prep(fp32, &e->P, e->stream), err);
   } else if (sh->kind == 3) {
-    HIPCHK(los_launch_window_prep(&e->P, e->stream), err);
+    const auto prep = e->form == LOS_FORM_FP64 ? los_launch_window_prep
+                      : fp32                   ? los_launch_window_prep_f32
+                                               : los_launch_window_prep_fma;
+    HIPCHK(prep(&e->P, e->stream), err);
   }
   return _SUCCESS_;
 }
@@ -1184,15 +1188,21 @@ int ensure_sweep(los_engine *e, const los_shape *sh, char *err)
 }
 
 // Device tables a k-lane shape needs (allocated outside any capture).
+// FP32 copy of the resident [jt][L][lm][x] table, made once per table upload.
+static int ensure_jk32(los_engine *e, char *err)
+{
+  if (e->dJk32 != nullptr) return _SUCCESS_;
+  HIPCHK(hipMalloc((void **)&e->dJk32, std::max<size_t>(1, e->nJk) * sizeof(float)), err);
+  HIPCHK(los_launch_round_j32(e->dJk, e->dJk32, (long)e->nJk, e->stream), err);
+  HIPCHK(hipStreamSynchronize(e->stream), err);
+  return _SUCCESS_;
+}
+
 int ensure_klane(los_engine *e, const los_shape *sh, char *err)
 {
   if (sh == nullptr || sh->kind != 2) return _SUCCESS_;
   const int fp32 = e->form == LOS_FORM_FP32C;
-  if (fp32 && e->dJk32 == nullptr) {
-    HIPCHK(hipMalloc((void **)&e->dJk32, std::max<size_t>(1, e->nJk) * sizeof(float)), err);
-    HIPCHK(los_launch_round_j32(e->dJk, e->dJk32, (long)e->nJk, e->stream), err);
-    HIPCHK(hipStreamSynchronize(e->stream), err);
-  }
+  if (fp32 && ensure_jk32(e, err)) return _FAILURE_;
   if (e->klane_form == e->form) return _SUCCESS_;
   if (e->dkixa) (void)hipFree(e->dkixa);
   if (e->dksrc) (void)hipFree(e->dksrc);
@@ -1237,6 +1247,7 @@ static void release_tables(los_engine *e, int kind)
 static int ensure_window(los_engine *e, const los_shape *sh, char *err)
 {
   if (sh == nullptr || sh->kind != 3) return _SUCCESS_;
+  if (e->form == LOS_FORM_FP32C && ensure_jk32(e, err)) return _FAILURE_;
   if (e->dwsrc) return _SUCCESS_;
   release_tables(e, 3);  // what a failed allocation left
   const size_t n = (size_t)e->P.k_npad * e->ntau;

@@ -46,6 +46,9 @@ extern "C" hipError_t los_launch_klane_exact(const los_params *P, int nlb, hipSt
 extern "C" hipError_t los_launch_window_prep(const los_params *P, hipStream_t s);
 extern "C" hipError_t los_launch_window_exact(const los_params *P, int kt, int nl, hipStream_t s);
 extern "C" hipError_t los_launch_window_fma(const los_params *P, int kt, int nl, hipStream_t s);
+extern "C" hipError_t los_launch_window_prep_fma(const los_params *P, hipStream_t s);
+extern "C" hipError_t los_launch_window_prep_f32(const los_params *P, hipStream_t s);
+extern "C" hipError_t los_launch_window_f32(const los_params *P, int kt, int nl, hipStream_t s);
 extern "C" int los_window_jrows(int NL, int Lmax, int m);
 extern "C" int los_window_rows_fit(int has_T, int has_P, int LmaxT, int LmaxP);
 extern "C" hipError_t los_launch_round_j32(const double *src, float *dst, long n, hipStream_t s);
@@ -151,7 +154,7 @@ struct los_engine {
   int2 *dwplan[LOS_TILE_SLOTS] = {};
   los_tile *dwtiles[LOS_TILE_SLOTS] = {};  // the tiles as dealt to the XCDs
   int wxcd[LOS_TILE_SLOTS][9] = {};        // first tile of each XCD
-  int *dwix = nullptr;                   // tables (both FP64 forms)
+  int *dwix = nullptr;                   // tables (FP32 values in the FP32 form)
   double *dwaj = nullptr, *dwsrc = nullptr;
   bool serving = false;                  // tiles are made per launch (the job server)
 

@@ -37,8 +37,10 @@
 // - Tiles of 64, 32 or 16 k3: the sparser the k3, the fewer share a window; the
 //   tuner picks (9,404 k3, T only, 48 l: 1.75, 0.89, 0.34 ms against the sweep
 //   kernel's 1.11 ms; 14,753 k3 up to 0.2/Mpc: 44.7, 26.6, 27.1 against 53.1 ms).
-// With FMA (11,178 k3, T+E+B, 96 l): 22.0, 14.3, 12.4 ms against 32.0 to 41.1 ms of
-// the sweep kernel's tiles.
+// The fast forms add a term to the running sums at a time, 32 steps a partial sum.
+// 11,178 k3, T+E+B, 96 l, tiles of 64, 32, 16 k3: with FMA 21.1, 15.1, 12.4 ms against
+// 22.7 to 29.5 ms of the sweep kernel's tiles; FP32-compensated 15.9, 9.9, 8.2 ms
+// against 17.7 to 20.4 ms (half the LDS and table bytes, as many instructions).
 //
 // Tables, by blocks of 64 sorted ranks (r = 64 rb + lane), so that a wave's
 // stream through the time steps is contiguous:
@@ -51,10 +53,47 @@
 #include <hip/hip_runtime.h>
 
 #include <climits>
+#include <type_traits>
 
 #include "los_device.h"
+#include "los_policy.h"
 
 typedef double win_d2 __attribute__((ext_vector_type(2)));
+
+// One value of a table of R at a lane's byte offset plus a wave-uniform one.
+template <class R>
+__device__ __forceinline__ R win_load(__amdgpu_buffer_rsrc_t r, unsigned lane, int off)
+{
+  if constexpr (sizeof(R) == 8)
+    return __builtin_bit_cast(R, __builtin_amdgcn_raw_buffer_load_b64(r, lane, off, 0));
+  else
+    return __builtin_bit_cast(R, __builtin_amdgcn_raw_buffer_load_b32(r, lane, off, 0));
+}
+
+// Forms: 0 plain FP64, 1 FP64 with FMA, 2 FP32-compensated.
+template <int FORM>
+using win_real = std::conditional_t<FORM == 2, float, double>;
+
+// Running sums of a pass: of the plain form as the reference adds them; of the
+// others over 32 time steps, then into the form's sum (of FP32 compensated).
+template <int FORM>
+struct WinAcc {
+  typedef std::conditional_t<FORM == 2, StreamFP32C, StreamFP64> Pol;
+  typename Pol::acc_t a;
+  win_real<FORM> p;
+  __device__ __forceinline__ void fold()
+  {
+    Pol::fold(a, p);
+    p = 0;
+  }
+  __device__ __forceinline__ double value() const { return Pol::value(a); }
+};
+template <>
+struct WinAcc<0> {
+  double s;
+  __device__ __forceinline__ void fold() {}
+  __device__ __forceinline__ double value() const { return s; }
+};
 
 // Raw buffer resource over `bytes` bytes at base (32-bit data, no swizzle): a load
 // adds the lane's byte offset and a wave-uniform one.
@@ -108,17 +147,26 @@ struct WinWave {
 // type y and field f goes to acc[j][y*NF + f], without the final 1/2 (SKIP: the
 // last of them is not wanted). src: the rank block's sources, NR*NF rows of 64
 // per step; field f of J row q is source row q*NF + f.
-template <int NR, int NF, int NT, bool SKIP, int NLB, int G>
-__device__ __forceinline__ void win_pass(const los_params &P, const WinWave &W, double *win,
-                                         int *xms, const int (&jt)[NT], int L0, const double *src,
-                                         double (&acc)[NLB][NT * NF])
+// The other forms: acc[j][f] is E (f = 0) and B of an l, or its only integral, and
+// the sources carry the trapezoid weight. The operations are those of the form's
+// sweep kernel in its order, so that both give the same bits from the same tables
+// (SKIP: no B sources into E; of one field, a product rounded before it is added).
+template <int FORM, int NR, int NF, int NT, bool SKIP, int NLB, int G, int NA,
+          class R = win_real<FORM>>
+__device__ __forceinline__ void win_pass(const los_params &P, const WinWave &W, R *win, int *xms,
+                                         const int (&jt)[NT], int L0, const R *src,
+                                         WinAcc<FORM> (&acc)[NLB][NA])
 {
-  constexpr int NLT = NLB * G, RL = NR * NT, ROWS = RL * NLT, NS = (ROWS + 3) / 4;
+  constexpr bool PLAIN = FORM == 0;
+  static_assert(NA == (PLAIN ? NT * NF : NF), "integrals of an l");
+  // a window is 32 points; 16 lanes (FP64) or 8 stage one with 16 bytes each
+  constexpr int LR = 2 * (int)sizeof(R), SR = 64 / LR, RB = 64 * (int)sizeof(R);
+  constexpr int NLT = NLB * G, RL = NR * NT, ROWS = RL * NLT, NS = (ROWS + SR - 1) / SR;
   const int lane = threadIdx.x;
 #pragma unroll
   for (int j = 0; j < NLB; ++j)
 #pragma unroll
-    for (int f = 0; f < NT * NF; ++f) acc[j][f] = 0;
+    for (int f = 0; f < NA; ++f) acc[j][f] = WinAcc<FORM>{};
 
   // Steps of each l, lane i searching for l number i of the wave (index_x falls
   // with t): before tsafe every row lives for every k3 of the tile, from tend on
@@ -163,43 +211,47 @@ __device__ __forceinline__ void win_pass(const los_params &P, const WinWave &W, 
   }
   if (tmax == 0) return;
 
-  // staged row s*4 + lane/16 = (l number) * RL + y * NR + q, x points
-  // 2 (lane%16) and the next
-  const unsigned rowx = (unsigned)P.X * 8u, typex = (unsigned)P.L_size * P.n_lm * rowx;
+  // staged row s*SR + lane/LR = (l number) * RL + y * NR + q, 16 bytes of x points
+  const unsigned rowx = (unsigned)P.X * sizeof(R), typex = (unsigned)P.L_size * P.n_lm * rowx;
   const __amdgpu_buffer_rsrc_t Jr = win_rsrc(P.Jk, P.Jk_bytes);
   unsigned voff[NS];
 #pragma unroll
   for (int s = 0; s < NS; ++s) {
-    const int ri = min(s * 4 + (lane >> 4), ROWS - 1);
+    const int ri = min(s * SR + lane / LR, ROWS - 1);
     const int li = ri / RL, yq = ri - li * RL, y = yq / NR, q = yq - y * NR;
     int lmr = W.lms[li];
     lmr = lmr < 0 ? W.lm0 : lmr;
-    if (s * 4 + (lane >> 4) < ROWS && (lane & 15) == 0)
+    if (s * SR + lane / LR < ROWS && lane % LR == 0)
       xms[ri] = P.xmin[((long)(NT > 1 && y ? jt[NT - 1] : jt[0]) * P.L_size + L0 + q) * P.n_lm +
                        lmr];
     voff[s] = (unsigned)(NT > 1 && y ? jt[NT - 1] : jt[0]) * typex +
-              (unsigned)((L0 + q) * P.n_lm + lmr) * rowx + (lane & 15) * 16u;
+              (unsigned)((L0 + q) * P.n_lm + lmr) * rowx + lane % LR * 16u;
   }
   const long tb = (long)W.rb * P.ntau * 64;
   const __amdgpu_buffer_rsrc_t Ir = win_rsrc(P.wix + tb, (unsigned)P.ntau * 256u),
-                               Ar = win_rsrc(P.waj + tb, (unsigned)P.ntau * 512u),
-                               Sr = win_rsrc(src, (unsigned)P.ntau * (NR * NF * 512u));
-  const unsigned rl4 = W.rl * 4u, rl8 = W.rl * 8u;
+                               Ar = win_rsrc((const R *)P.waj + tb, (unsigned)P.ntau * RB),
+                               Sr = win_rsrc(src, (unsigned)P.ntau * (NR * NF * RB));
+  const unsigned rl4 = W.rl * 4u, rlr = W.rl * (unsigned)sizeof(R);
   int ixn = 0;
-  double an = 0, svn[NF][NR];
+  R an = 0, svn[NF][NR];
   // index_x, a_J and the sources of step t
   auto load = [&](int t) {
     ixn = (int)__builtin_amdgcn_raw_buffer_load_b32(Ir, rl4, t * 256, 0);
-    an = __builtin_bit_cast(double, __builtin_amdgcn_raw_buffer_load_b64(Ar, rl8, t * 512, 0));
-    const int so = t * (NR * NF * 512);
+    an = win_load<R>(Ar, rlr, t * RB);
+    const int so = t * (NR * NF * RB);
 #pragma unroll
     for (int q = 0; q < NR; ++q)
 #pragma unroll
       for (int f = 0; f < NF; ++f) {
-        const int o = (q * NF + f) * 512, hi = o & ~4095;
-        svn[f][q] = __builtin_bit_cast(
-            double, __builtin_amdgcn_raw_buffer_load_b64(Sr, rl8 + (o - hi), so + hi, 0));
+        const int o = (q * NF + f) * RB, hi = o & ~4095;
+        svn[f][q] = win_load<R>(Sr, rlr + (o - hi), so + hi);
       }
+  };
+  auto fold = [&]() {
+#pragma unroll
+    for (int j = 0; j < NLB; ++j)
+#pragma unroll
+      for (int f = 0; f < NA; ++f) acc[j][f].fold();
   };
 
   int i = 0;
@@ -215,89 +267,124 @@ __device__ __forceinline__ void win_pass(const los_params &P, const WinWave &W, 
 #pragma unroll
       for (int s = 0; s < NS; ++s)
         w[s] = __builtin_bit_cast(
-            win_d2, __builtin_amdgcn_raw_buffer_load_b128(Jr, voff[s], x0 * 8, 0));
+            win_d2, __builtin_amdgcn_raw_buffer_load_b128(Jr, voff[s], x0 * (int)sizeof(R), 0));
 #pragma unroll
       for (int s = 0; s < NS; ++s)
-        if (s * 4 + 3 < ROWS || s * 4 + (lane >> 4) < ROWS) ((win_d2 *)win)[s * 64 + lane] = w[s];
+        if (s * SR + SR - 1 < ROWS || s * SR + lane / LR < ROWS) ((win_d2 *)win)[s * 64 + lane] = w[s];
       __builtin_amdgcn_sched_barrier(0);
     }
     win_fence();
     const int te = min(max(nbt, bt + 1), tmax);
     for (int t = bt; t < te; ++t) {
       const int ix = ixn;
-      const double a = an, ar = 1 - a;
-      double sv[NF][NR];
+      const R a = an;
+      R sv[NF][NR];
 #pragma unroll
       for (int f = 0; f < NF; ++f)
 #pragma unroll
         for (int q = 0; q < NR; ++q) sv[f][q] = svn[f][q];
       const int tn = t + 1 < te ? t + 1 : nbt;
       if (tn < tmax) load(tn);
-      const double dt = win_uniform(P.dtau, t);
       const int cell = ix - x0;
-      const double *wl = win + W.grp * (RL * LOS_WIN_W) + cell;
+      const R *wl = win + W.grp * (RL * LOS_WIN_W) + cell;
       if (!partial || (unsigned)cell < LOS_WIN_W - 1) {
 #pragma unroll
         for (int j = 0; j < NLB; ++j) {
           if (t >= tend[j]) continue;
           const bool safe = t < tsafe[j];
+          if constexpr (PLAIN) {
+            const double ar = 1 - a, dt = win_uniform(P.dtau, t);
 #pragma unroll
-          for (int y = 0; y < NT; ++y) {
-            __builtin_amdgcn_sched_barrier(0);
-            const double *wj = wl + (j * G * RL + y * NR) * LOS_WIN_W;
-            double v[NF];
-            if (safe) {
-              // the sum starts with its first term, not with 0 + it: that can only
-              // turn a +0 into a -0, which adds the same to acc (never -0 itself)
+            for (int y = 0; y < NT; ++y) {
+              __builtin_amdgcn_sched_barrier(0);
+              const double *wj = wl + (j * G * RL + y * NR) * LOS_WIN_W;
+              double v[NF];
+              if (safe) {
+                // the sum starts with its first term, not with 0 + it: that can only
+                // turn a +0 into a -0, which adds the same to acc (never -0 itself)
 #pragma unroll
-              for (int q = 0; q < NR; ++q) {
-                const double Jv = a * wj[q * LOS_WIN_W] + ar * wj[q * LOS_WIN_W + 1];
+                for (int q = 0; q < NR; ++q) {
+                  const double Jv = a * wj[q * LOS_WIN_W] + ar * wj[q * LOS_WIN_W + 1];
 #pragma unroll
-                for (int f = 0; f < NF; ++f)
-                  if (!(SKIP && y == NT - 1 && f == NF - 1))
-                    v[f] = q == 0 ? Jv * sv[f][q] : v[f] + Jv * sv[f][q];
+                  for (int f = 0; f < NF; ++f)
+                    if (!(SKIP && y == NT - 1 && f == NF - 1))
+                      v[f] = q == 0 ? Jv * sv[f][q] : v[f] + Jv * sv[f][q];
+                }
+              } else {
+                // some row is dead (index_x < index_xmin_J) for some k3: J = 0 there
+                const int *xj = xms + W.grp * RL + j * (G * RL) + y * NR;
+#pragma unroll
+                for (int q = 0; q < NR; ++q) {
+                  double Jv = a * wj[q * LOS_WIN_W] + ar * wj[q * LOS_WIN_W + 1];
+                  Jv = ix >= xj[q] ? Jv : 0.;
+#pragma unroll
+                  for (int f = 0; f < NF; ++f)
+                    if (!(SKIP && y == NT - 1 && f == NF - 1))
+                      v[f] = q == 0 ? Jv * sv[f][q] : v[f] + Jv * sv[f][q];
+                }
               }
-            } else {
-              // some row is dead (index_x < index_xmin_J) for some k3: J = 0 there
-              const int *xj = xms + W.grp * RL + j * (G * RL) + y * NR;
 #pragma unroll
-              for (int q = 0; q < NR; ++q) {
-                double Jv = a * wj[q * LOS_WIN_W] + ar * wj[q * LOS_WIN_W + 1];
-                Jv = ix >= xj[q] ? Jv : 0.;
-#pragma unroll
-                for (int f = 0; f < NF; ++f)
-                  if (!(SKIP && y == NT - 1 && f == NF - 1))
-                    v[f] = q == 0 ? Jv * sv[f][q] : v[f] + Jv * sv[f][q];
-              }
+              for (int f = 0; f < NF; ++f)
+                if (!(SKIP && y == NT - 1 && f == NF - 1)) acc[j][y * NF + f].s += v[f] * dt;
             }
+          } else {
+            __builtin_amdgcn_sched_barrier(0);
+            const R *wj = wl + j * G * RL * LOS_WIN_W;
+            const int *xj = xms + W.grp * RL + j * (G * RL);
+            auto fma = [](R x, R y, R z) { return __builtin_elementwise_fma(x, y, z); };
+            auto node = [&](int row, bool live) {
+              const R j0 = wj[row * LOS_WIN_W], j1 = wj[row * LOS_WIN_W + 1];
+              const R v = fma(a, j0 - j1, j1);
+              return live || ix >= xj[row] ? v : (R)0;
+            };
+            auto sum = [&](bool live) {
+#pragma clang fp contract(off)
 #pragma unroll
-            for (int f = 0; f < NF; ++f)
-              if (!(SKIP && y == NT - 1 && f == NF - 1)) acc[j][y * NF + f] += v[f] * dt;
+              for (int q = 0; q < NR; ++q) {
+                const R Je = node(q, live);
+                R &pE = acc[j][0].p, &pB = acc[j][NA - 1].p;
+                if constexpr (NT == 1) {
+                  pE = SKIP ? pE + Je * sv[0][q] : fma(Je, sv[0][q], pE);
+                } else {
+                  const R Jm = node(NR + q, live), sE = sv[0][q], sB = sv[NF - 1][q];
+                  pE += SKIP ? Je * sE : fma(Je, sE, Jm * sB);
+                  pB += fma(Je, sB, -(Jm * sE));
+                }
+              }
+            };
+            if (safe)
+              sum(true);
+            else
+              sum(false);
           }
         }
       }
+      // the same 32 steps a sum as in the sweep kernel, once all windows of the
+      // last of them are done
+      if (!PLAIN && (t & 31) == 31 && tn != t) fold();
     }
     win_fence();
     bt = nbt;
     by = nby;
   }
+  fold();
 }
 
 // One wave: the integrals of one field set and its outputs. Set 1: T, NLT l
 // numbers; set 0: E and B, half as many with twice the rows (EE: the E and B
 // sources into E and B; EB: the E sources into B and, for m != 0, the B sources
 // into E).
-template <int NR, int NLT, int G>
-__device__ __forceinline__ void win_item(const los_params &P, const WinWave &W, double *win,
+template <int FORM, int NR, int NLT, int G, class R = win_real<FORM>>
+__device__ __forceinline__ void win_item(const los_params &P, const WinWave &W, R *win,
                                          int *xms, const los_tile *tile, int set, int mi)
 {
   const int m = P.m_of_mi[mi];
   const int L0 = (set ? P.LmaxT : P.LmaxP) - NR + 1;
   const bool two = !set && P.has_B;
-  const double *src =
-      P.wsrc + P.wsrc_off[set][mi] + (long)W.rb * P.ntau * (NR * (two ? 2 : 1)) * 64;
+  const R *src =
+      (const R *)P.wsrc + P.wsrc_off[set][mi] + (long)W.rb * P.ntau * (NR * (two ? 2 : 1)) * 64;
   auto store = [&](auto &acc) {
-    constexpr int NLB = sizeof(acc) / sizeof(acc[0]), N = sizeof(acc[0]) / sizeof(double);
+    constexpr int NLB = sizeof(acc) / sizeof(acc[0]), N = sizeof(acc[0]) / sizeof(WinAcc<FORM>);
     const int i = threadIdx.x & (64 / G - 1);
     const int pos0 = win_uniform(&tile->pos0, 0), npos = win_uniform(&tile->npos, 0);
     const los_job job = P.jobs[win_uniform(P.pos_job, pos0)];
@@ -319,7 +406,8 @@ __device__ __forceinline__ void win_item(const los_params &P, const WinWave &W, 
       };
       double h[N];
 #pragma unroll
-      for (int f = 0; f < N; ++f) h[f] = acc[j][f] * 0.5;
+      for (int f = 0; f < N; ++f)
+        h[f] = acc[j][f].value() * 0.5;
       if (N == 1) {
         *(set ? oT : oE) = scaled(set ? h[0] : h[0] + 0.);
       } else {
@@ -329,17 +417,20 @@ __device__ __forceinline__ void win_item(const los_params &P, const WinWave &W, 
     }
   };
   if (two && P.jEB >= 0) {
-    double acc[NLT / 2 / G][4];
+    WinAcc<FORM> acc[NLT / 2 / G][FORM == 0 ? 4 : 2];
     const int jt[2] = {P.jEE, P.jEB};
     if (m != 0)
-      win_pass<NR, 2, 2, false, NLT / 2 / G, G>(P, W, win, xms, jt, L0, src, acc);
+      win_pass<FORM, NR, 2, 2, false, NLT / 2 / G, G>(P, W, win, xms, jt, L0, src, acc);
     else
-      win_pass<NR, 2, 2, true, NLT / 2 / G, G>(P, W, win, xms, jt, L0, src, acc);
+      win_pass<FORM, NR, 2, 2, true, NLT / 2 / G, G>(P, W, win, xms, jt, L0, src, acc);
     store(acc);
   } else {
-    double acc[NLT / G][1];
+    WinAcc<FORM> acc[NLT / G][1];
     const int jt[1] = {set ? P.jTT : P.jEE};
-    win_pass<NR, 1, 1, false, NLT / G, G>(P, W, win, xms, jt, L0, src, acc);
+    if (FORM == 0 || set)
+      win_pass<FORM, NR, 1, 1, false, NLT / G, G>(P, W, win, xms, jt, L0, src, acc);
+    else
+      win_pass<FORM, NR, 1, 1, FORM != 0, NLT / G, G>(P, W, win, xms, jt, L0, src, acc);
     store(acc);
   }
 }
@@ -349,15 +440,14 @@ __device__ __forceinline__ void win_item(const los_params &P, const WinWave &W, 
 // XCD's tiles, costliest first, then the l groups, so that the waves running
 // together read the sources of a few neighbouring tiles and the same stretch
 // of their J rows through the XCD's L2.
-// FMA tells the unit that instantiates it apart: the plain FP64 form (compiled
-// without contraction) or the FP64 form with FMA.
-template <bool FMA, int NL, int NLT, int G>
+template <int FORM, int NL, int NLT, int G>
 __global__ void __launch_bounds__(64) __attribute__((amdgpu_waves_per_eu(2)))
 los_window(los_params P)
 {
+  typedef win_real<FORM> R;
   constexpr int KT = 64 / G;
-  __shared__ alignas(16) double win[NL * NLT * LOS_WIN_W];  // windows of the wave's rows
-  __shared__ int xms[NL * NLT];                             // and their first live x points
+  __shared__ alignas(16) R win[NL * NLT * LOS_WIN_W];  // windows of the wave's rows
+  __shared__ int xms[NL * NLT];                        // and their first live x points
   const int xcd = blockIdx.x & 7;
   int q = blockIdx.x >> 3;
   const int nt = P.xcd_tile[xcd + 1] - P.xcd_tile[xcd];
@@ -386,11 +476,11 @@ los_window(los_params P)
   W.plan = (const int *)(P.wplan + win_uniform(P.wplan_off, tile));
   const int nr = win_jrows(NL, set ? P.LmaxT : P.LmaxP, P.m_of_mi[mi]);
   if (nr == NL)
-    win_item<NL, NLT, G>(P, W, win, xms, P.tiles + tile, set, mi);
+    win_item<FORM, NL, NLT, G>(P, W, win, xms, P.tiles + tile, set, mi);
   else if (NL > 1 && nr == NL - 1)
-    win_item<(NL > 1 ? NL - 1 : 1), NLT, G>(P, W, win, xms, P.tiles + tile, set, mi);
+    win_item<FORM, (NL > 1 ? NL - 1 : 1), NLT, G>(P, W, win, xms, P.tiles + tile, set, mi);
   else if (NL > 2)
-    win_item<(NL > 2 ? NL - 2 : 1), NLT, G>(P, W, win, xms, P.tiles + tile, set, mi);
+    win_item<FORM, (NL > 2 ? NL - 2 : 1), NLT, G>(P, W, win, xms, P.tiles + tile, set, mi);
 }
 
 // Whether the window kernels cover a batch's multipoles: they have instances
@@ -405,7 +495,7 @@ static inline bool window_rows_fit(int has_T, int has_P, int LmaxT, int LmaxP)
 
 // P->tiles / P->xcd_tile: tiles of at most 64/G positions; P->wgrp: groups of NLT
 // (l,m) offsets, of NLT/2 for E and B with B sources.
-template <bool FMA, int NLT, int G>
+template <int FORM, int NLT, int G>
 static hipError_t launch_window(const los_params *P, hipStream_t s)
 {
   if (P->n_pos == 0 || P->n_lm_max == 0) return hipSuccess;
@@ -422,7 +512,7 @@ static hipError_t launch_window(const los_params *P, hipStream_t s)
   switch ((P->LmaxT > P->LmaxP ? P->LmaxT : P->LmaxP) + 1) {
 #define LOS_WN(n)                                                                              \
   case n:                                                                                      \
-    hipLaunchKernelGGL((los_window<FMA, n, NLT, G>), dim3((unsigned)grid), dim3(64), 0, s, *P); \
+    hipLaunchKernelGGL((los_window<FORM, n, NLT, G>), dim3((unsigned)grid), dim3(64), 0, s, *P); \
     break;
     LOS_WN(1) LOS_WN(2) LOS_WN(3) LOS_WN(4) LOS_WN(5) LOS_WN(6) LOS_WN(7) LOS_WN(8)
 #undef LOS_WN
@@ -432,13 +522,102 @@ static hipError_t launch_window(const los_params *P, hipStream_t s)
 }
 
 // kt fine k3 and nl (l,m) offsets per wave
-template <bool FMA>
+template <int FORM>
 static hipError_t launch_window(const los_params *P, int kt, int nl, hipStream_t s)
 {
   switch (kt * 64 + nl) {
-    case 64 * 64 + 8: return launch_window<FMA, 8, 1>(P, s);
-    case 32 * 64 + 8: return launch_window<FMA, 8, 2>(P, s);
-    case 16 * 64 + 8: return launch_window<FMA, 8, 4>(P, s);
+    case 64 * 64 + 8: return launch_window<FORM, 8, 1>(P, s);
+    case 32 * 64 + 8: return launch_window<FORM, 8, 2>(P, s);
+    case 16 * 64 + 8: return launch_window<FORM, 8, 4>(P, s);
     default: return hipErrorInvalidValue;
   }
+}
+
+// The tables of the window kernels. A workgroup makes 64 ranks x 64 time steps:
+// it reads the sources along tau (their layout in HBM) and writes along the
+// ranks through an LDS transpose. The fast forms' sources carry the
+// trapezoid weight.
+template <int FORM, class R = win_real<FORM>>
+__global__ void __launch_bounds__(256) los_window_prep(los_params P)
+{
+  __shared__ R tile[64][65];
+  __shared__ long r_off[64];
+  __shared__ int r_nc[64];
+  __shared__ double r_aw[64], r_bw[64], r_ca[64], r_cb[64], r_h[64];
+  const int rb = blockIdx.x, r0 = rb * 64, t0 = blockIdx.y * 64;
+  const int tid = threadIdx.x, lane = tid & 63, grp = tid >> 6;
+  double kf = 0;
+  {
+    const int r = min(r0 + lane, P.F - 1);
+    const int f = P.korder[r];
+    kf = P.kf[f];
+    if (tid < 64) {
+      const los_pair pr = P.pairs[P.fpair[f]];
+      const int br = P.fbr[f];
+      const double *kc = P.kc + pr.kc_off;
+      const double ks = P.kf[P.fsrc[f]];
+      const double h = kc[br + 1] - kc[br];
+      const double bw = (ks - kc[br]) / h;
+      const double aw = 1 - bw;
+      r_off[tid] = pr.src_off + (long)br * P.ntau;
+      r_nc[tid] = pr.nc;
+      r_h[tid] = h;
+      r_aw[tid] = aw;
+      r_bw[tid] = bw;
+      r_ca[tid] = aw * aw * aw - aw;
+      r_cb[tid] = bw * bw * bw - bw;
+    }
+  }
+  for (int i = grp; i < 64; i += 4) {
+    const int t = t0 + i;
+    if (t >= P.ntau) break;
+    const double x = kf * P.t0mt[t];
+    const int ix = (int)(x / P.xx_step);
+    const long o = ((long)rb * P.ntau + t) * 64 + lane;
+    P.wix[o] = ix;
+    ((R *)P.waj)[o] = (R)((P.xx[ix + 1] - x) / P.xx_step);
+  }
+  const int tr = min(t0 + lane, P.ntau - 1);
+  const double dt = P.dtau[tr];
+  __syncthreads();
+  for (int set = 0; set < 2; ++set) {
+    if (set ? !P.has_T : !(P.has_E || P.has_B)) continue;
+    const int Lmax = set ? P.LmaxT : P.LmaxP, nf = set || !P.has_B ? 1 : 2;
+    for (int mi = 0; mi < P.m_size; ++mi) {
+      const int m = P.m_of_mi[mi], nr = win_jrows(P, set, m), rows = nr * nf;
+      R *out = (R *)P.wsrc + P.wsrc_off[set][mi] + (long)rb * P.ntau * rows * 64;
+      for (int row = 0; row < rows; ++row) {
+        const int L = Lmax - nr + 1 + row / nf;
+        const bool live = L >= m;
+        const int tp = !live ? 0 : set ? P.srcT[L][mi] : row % nf ? P.srcB[L][mi] : P.srcE[L][mi];
+#pragma unroll 4
+        for (int i = grp; i < 64; i += 4) {
+          const double *S = P.src + r_off[i] + (long)tp * r_nc[i] * P.ntau + tr;
+          double v;
+          if (P.cubic_k3) {
+            const double *D = P.dd + (S - P.src);
+            v = r_aw[i] * S[0] + r_bw[i] * S[P.ntau] +
+                (r_ca[i] * D[0] + r_cb[i] * D[P.ntau]) * r_h[i] * r_h[i] / 6.0;
+          } else {
+            v = r_aw[i] * S[0] + r_bw[i] * S[P.ntau];
+          }
+          if (FORM != 0) v = v * dt;
+          tile[i][lane] = (R)(live ? v : 0.);
+        }
+        __syncthreads();
+        for (int i = grp; i < 64; i += 4)
+          if (t0 + i < P.ntau) out[((long)(t0 + i) * rows + row) * 64 + lane] = tile[lane][i];
+        __syncthreads();
+      }
+    }
+  }
+}
+
+template <int FORM>
+static hipError_t launch_window_prep(const los_params *P, hipStream_t s)
+{
+  if (P->F == 0 || P->ntau == 0) return hipSuccess;
+  const dim3 grid((unsigned)(P->k_npad / 64), (unsigned)((P->ntau + 63) / 64));
+  hipLaunchKernelGGL(los_window_prep<FORM>, grid, dim3(256), 0, s, *P);
+  return hipGetLastError();
 }

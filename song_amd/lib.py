@@ -474,7 +474,7 @@ class Engine:
     def set_shape(self, form: int, kind: int, nk: int = 64, ch: int = 0,
                   persistent: int = 0) -> None:
         """Kernel of a form. Plain FP64: kind 0 (workgroup per k3), 1 (sweep), 2 (k-lane)
-        or 3 (window: nk k3 and ch l a wave); fast forms: kind 0 stream (nk, ch, persistent), 1 sweep (nk), 2 k-lane."""
+        or 3 (window: nk k3 and ch l a wave); fast forms: kind 0 stream (nk, ch, persistent), 1 sweep (nk), 2 k-lane, 3 window."""
         self._call("los_engine_set_shape", form, kind, nk, ch, persistent)
 
     def get_shape(self, form: int):

@@ -1,5 +1,6 @@
 """The window kernels (one fine k3 per lane, J windows in LDS) against the CPU oracle, the plain
-FP64 form bit for bit and the FMA-FP64 form at its bar, where they can go wrong: every count of
+FP64 form bit for bit and the FMA-FP64 form at its bar, and the FP32-compensated form against the
+sweep kernel bit for bit, where they can go wrong: every count of
 source multipoles L, rows below m, fields with fewer L than the other, T or E alone, odd l
 counts against the groups of 8 and 4, k3 counts that leave partial tiles, one step over several
 windows, J rows with an index_xmin_J of their own, and a batch whose k3 lie too far apart.
@@ -77,6 +78,42 @@ def test_window_equals_oracle(name, oracle):
         assert np.count_nonzero(ref) > 0.1 * ref.size
 
 
+def _same_as_sweep(cfg, overrides=()):
+    s = L.Scenario(cfg)
+    for o in overrides:
+        s.override_J(*o)
+    s.prepare()
+    eng = L.Engine(0)
+    eng.set_form(L.FORM_FP32C)
+    eng.load(s)
+    eng.set_shape(L.FORM_FP32C, 1, 2, 1, 0)
+    eng.run()
+    eng.store(s)
+    ref, ran = s.gather(), []
+    for kt in (64, 32, 16):
+        print(f"tile of {kt}", flush=True)
+        try:
+            eng.set_shape(L.FORM_FP32C, 3, kt, 8, 0)
+        except L.LosError:
+            continue
+        eng.run()
+        eng.store(s)
+        assert np.array_equal(s.gather(), ref), f"tile of {kt}"
+        ran.append(kt)
+    eng.close()
+    s.close()
+    assert 16 in ran
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("tau_size", [31, 32, 33, 70])
+@pytest.mark.parametrize("name", list(CASES))
+def test_fp32_window_equals_sweep(name, tau_size):
+    """Counts of time steps about the 32 of a partial sum."""
+    print(f"case {name} {tau_size} steps", flush=True)
+    _same_as_sweep(L.Config(**dict(CASES[name], tau_size=tau_size)))
+
+
 @pytest.mark.gpu
 def test_window_rows_with_their_own_first_point(oracle):
     """J rows of one l whose first stored points are far apart: the skip holds row by row."""
@@ -92,6 +129,7 @@ def test_window_rows_with_their_own_first_point(oracle):
     s.close()
     _, ran = _run(cfg, oracle, over)
     assert 16 in ran
+    _same_as_sweep(cfg, over)
 
 
 @pytest.mark.gpu
