@@ -14,8 +14,8 @@
 // below index_xmin_J (source/transfer2.c:2232) is a select on the
 // interpolated J. No LDS and no barriers: waves are independent.
 //
-// Bound by the J rows it fetches. Two things keep a wave from fetching what it
-// need not: a lane none of whose rows lives at the element's index_x is given an
+// Bound by the J rows it fetches. In FP64 two things keep a wave from fetching what
+// it need not: a lane none of whose rows lives at the element's index_x is given an
 // offset out of the table (64 l span a wide range of first live points), and the
 // row registers outlive the step (index_x stays for several early steps). Plain
 // FP64, tiles of one k3: 3,098 k3 x 251 steps x 37 l x m = 0, 2: 1.87 to 1.18 ms;
@@ -518,10 +518,13 @@ __device__ __forceinline__ void sweep_item(const los_params &P, int xcd, int q, 
   int fl = f[0];  // this lane's element (lanes below NK)
 #pragma unroll
   for (int j = 1; j < NK; ++j) fl = li == j ? f[j] : fl;
-  // a lane whose rows are all dead at the element's index_x reads nothing (an
-  // offset out of the resource's range gives 0); `held` is the index_x in the row
-  // registers, which outlives the step
-  const int xml = active ? P.min_xmin[lm] : INT_MAX;
+  // FP64: a lane whose rows are all dead at the element's index_x reads nothing (an
+  // offset out of the resource's range gives 0), and the rows outlive the step.
+  // FP32 rows are half the bytes: there the select before each load costs more
+  // (one k3 a tile: 2,444 k3 x 230 steps x 30 l 296 us without, 311 with it).
+  // held: the index_x in the row registers.
+  constexpr bool F64 = sizeof(R) == 8;
+  const int xml = F64 && active ? P.min_xmin[lm] : INT_MAX;
   int held = -1;
   SweepIXA<R> nxt{};
   if (li < NK && tend > 0) nxt = ixa[(long)fl * P.ntau];
@@ -549,9 +552,10 @@ __device__ __forceinline__ void sweep_item(const los_params &P, int xcd, int q, 
       // usually share it), so one set of row registers serves the tile
 #pragma unroll
       for (int j = 0; j < NK; ++j) {
-        if (ix[j] != held) {
+        if ((!F64 && j == 0) || ix[j] != held) {
           held = ix[j];
-          const unsigned ox = (unsigned)ix[j] * xstep, lo = held >= xml ? lane : SWEEP_OUT;
+          const unsigned ox = (unsigned)ix[j] * xstep,
+                         lo = !F64 || held >= xml ? lane : SWEEP_OUT;
 #pragma unroll
           for (int L = 0; L < NL; ++L) {
             if (m > L) continue;
