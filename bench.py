@@ -461,8 +461,8 @@ def cl2_bench(args, cfg):
                    "ms_TT": res["TT"][1], "ms_EE": res["EE"][1]},
         "roofline": {"bound": "hbm", "achieved": achieved, "peak": HBM_PEAK_GBS, "unit": "GB/s",
                      "frac": achieved / HBM_PEAK_GBS,
-                     "traffic": measured_traffic("cl2", "los_cl2_partial + los_cl2_finish"),
-                     "kernel": "los_cl2_partial + los_cl2_finish",
+                     "traffic": measured_traffic("cl2", "los_cl2_weights + los_cl2_partial + los_cl2_finish"),
+                     "kernel": "los_cl2_weights + los_cl2_partial + los_cl2_finish",
                      "kernel_ms": ms_tot / 2, "alg_bytes": alg_bytes / 2},
     }
     if not args.no_cpu:
